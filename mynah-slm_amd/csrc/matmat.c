@@ -20,41 +20,93 @@ static long env_long(const char *name, long dflt) {
     return (e != NULL && e[0] != '\0') ? strtol(e, NULL, 10) : dflt;
 }
 
+/* How an exact GEMM runs: kw waves share each 16-row group of a 64 x 64 tile
+ * and hand its running totals on, unit by unit, inside the workgroup; nz
+ * splits of the super-blocks (gridDim.z) whose later unit sums go through
+ * memory and are folded in order afterwards (mynah_gemm_fold). */
+typedef struct {
+    uint32_t kw, nz;
+} gemm_split;
+
+/* Nanoseconds per column step and SIMD with w waves on it, measured on MI355X
+ * (Q4_K 512 .. 9728 rows x 2048 / 2560 columns, 512 and 2047 tokens), by kw
+ * (1, 2, 4) and w. The bound is 28.7 at 2 or 4 waves, 34 at 3, 43.7 at 1;
+ * waves that share row groups keep in step through two barriers more per
+ * unit, so kw > 1 costs where a launch has waves enough without it
+ * (9728 x 2560, 2047 tokens: 1600 us with kw 1, 1647 with 2, 1946 with 4) and
+ * pays where it has not (2048 x 2048, 512 tokens: 111, 90 and 86 us). */
+static const double gemm_step_ns[3][5] = {{0.0, 54.0, 37.8, 37.3, 33.0},
+                                          {0.0, 0.0, 44.0, 0.0, 36.0},
+                                          {0.0, 0.0, 0.0, 0.0, 41.0}};
+
+/* The (kw, nz) of least estimated time. A CU holds 16 waves of these kernels,
+ * 4 / kw workgroups; a launch runs in rounds of resident workgroups, each
+ * round's length set by its longest split (in rounds of kw units) and the
+ * waves per SIMD it leaves; a split costs the fold's traffic (each unit sum
+ * past the first split written and read, about 4.5 TB/s) and its launch.
+ * cap: most splits. */
+static gemm_split gemm_plan(uint64_t tiles, uint32_t units, uint64_t outputs, uint32_t cus,
+                            uint32_t max_kw, uint32_t cap) {
+    gemm_split best = {1, 1};
+    double best_ns = 0.0;
+    for (uint32_t kw = 1, i = 0; kw <= max_kw && kw <= units; kw *= 2u, i++) {
+        const uint64_t slots = (uint64_t)cus * (4u / kw);
+        for (uint32_t nz = 1; nz <= cap && nz <= units; nz++) {
+            if (nz > 1 && tiles * (nz - 1u) >= slots) break;
+            const uint32_t per = (units + nz - 1u) / nz;
+            const double steps = 256.0 * (double)((per + kw - 1u) / kw);
+            uint64_t left = tiles * nz;
+            const uint64_t full = left / slots;
+            double ns = (double)full * steps * 4.0 * gemm_step_ns[i][4];
+            left -= full * slots;
+            if (left > 0) {
+                const uint32_t w = kw * (uint32_t)((left + cus - 1u) / cus);
+                ns += steps * (double)w * gemm_step_ns[i][w];
+            }
+            if (nz > 1)
+                ns += 4000.0 + (double)outputs * 8.0 * (double)(units - units / nz + 1u) / 4500.0;
+            if (best_ns == 0.0 || ns < best_ns) {
+                best_ns = ns;
+                best.kw = kw;
+                best.nz = nz;
+            }
+        }
+    }
+    return best;
+}
+
 /* The exact GEMM with its products on MFMA (gemm_mfma.hip): the default;
  * MYNAH_GEMM_MFMA=0 runs the VALU kernels of gemm_exact.hip instead (same
- * bits). A launch of at most one 64 x 64 tile per CU splits the
- * super-blocks over gridDim.z, up to MYNAH_GEMM_WGS_PER_CU (default 4)
- * workgroups per CU (MYNAH_GEMM_SPLIT=0 never, N at most N ways), and folds
- * the first split's running total and the later per-super-block sums in
- * order afterwards (mynah_gemm_fold). */
+ * bits). MYNAH_GEMM_SPLIT=0 never splits over gridDim.z, N at most N ways;
+ * MYNAH_GEMM_KW=1|2|4 forces kw. */
 static int gemm_mfma_launch(mynah_device *d, int type, int ord, const void *w, size_t rows,
                             size_t cols, size_t rb, const float *x, float *y, size_t tokens,
                             const float *res, hipStream_t stream) {
+    /* Q6_K sums in one order either way. */
     static const int kid[2][4] = {
-        {MYNAH_K_Q4K_GEMM_MFMA, MYNAH_K_Q5K_GEMM_MFMA, MYNAH_K_Q6K_GEMM_MFMA,
-         MYNAH_K_Q80_GEMM_MFMA},
-        {MYNAH_K_Q4K_GEMM_MV_MFMA, MYNAH_K_Q5K_GEMM_MV_MFMA, MYNAH_K_Q6K_GEMM_MV_MFMA,
-         MYNAH_K_Q80_GEMM_MV_MFMA}};
+        {MYNAH_K_Q4K_GEMM_MFMA1, MYNAH_K_Q5K_GEMM_MFMA1, MYNAH_K_Q6K_GEMM_MFMA1,
+         MYNAH_K_Q80_GEMM_MFMA1},
+        {MYNAH_K_Q4K_GEMM_MV_MFMA1, MYNAH_K_Q5K_GEMM_MV_MFMA1, MYNAH_K_Q6K_GEMM_MFMA1,
+         MYNAH_K_Q80_GEMM_MV_MFMA1}};
     const int ti = type == MYNAH_Q4_K ? 0 : type == MYNAH_Q5_K ? 1 : type == MYNAH_Q6_K ? 2 : 3;
     const uint32_t units = (uint32_t)(cols / 256);
     const unsigned gx = (unsigned)((rows + 63) / 64), gy = (unsigned)((tokens + 63) / 64);
-    const uint64_t tiles = (uint64_t)gx * gy;
-    uint32_t nz = 1;
-    const char *env = getenv("MYNAH_GEMM_SPLIT");
-    const long cap = env ? strtol(env, NULL, 10) : 64;
-    const long per_cu = env_long("MYNAH_GEMM_WGS_PER_CU", 4);
-    const uint64_t want = (uint64_t)(per_cu > 0 ? per_cu : 1) * (uint64_t)d->cus;
-    if (!(ord == 1 && type == MYNAH_Q8_0) && cap > 1 && tiles <= (uint64_t)d->cus) {
-        nz = (uint32_t)((want + tiles - 1) / tiles);
-        if (nz > units) nz = units;
-        if (nz > (uint32_t)cap) nz = (uint32_t)cap;
+    gemm_split p = {1, 1};
+    if (!(ord == 1 && type == MYNAH_Q8_0)) {
+        const long cap = env_long("MYNAH_GEMM_SPLIT", 64), kw = env_long("MYNAH_GEMM_KW", 0);
+        p = gemm_plan((uint64_t)gx * gy, units, (uint64_t)rows * tokens, (uint32_t)d->cus, 4u,
+                      cap > 1 ? (uint32_t)cap : 1u);
+        if (kw == 1 || kw == 2 || kw == 4) p.kw = (uint32_t)kw;
     }
+    const uint32_t nz = p.nz;
+    const int kernel = kid[ord][ti] + (p.kw == 4 ? 2 : p.kw == 2 ? 1 : 0);
+    const unsigned block = 256u * p.kw;
     uint32_t r32 = (uint32_t)rows, c32 = (uint32_t)cols, t32 = (uint32_t)tokens,
              rb32 = (uint32_t)rb;
     if (nz <= 1) {
         float *part = NULL;
         void *args[] = {&w, &x, &y, &r32, &c32, &t32, &rb32, &res, &part};
-        return mynah_launch3(d, kid[ord][ti], gx, gy, 1, 256, 0, stream, args);
+        return mynah_launch3(d, kernel, gx, gy, 1, block, 0, stream, args);
     }
     const size_t n = rows * tokens, bytes = (size_t)units * n * sizeof(float);
     float *part = NULL;
@@ -65,7 +117,7 @@ static int gemm_mfma_launch(mynah_device *d, int type, int ord, const void *w, s
         return -1;
     }
     void *args[] = {&w, &x, &y, &r32, &c32, &t32, &rb32, &res, &part};
-    int rc = mynah_launch3(d, kid[ord][ti], gx, gy, nz, 256, 0, stream, args);
+    int rc = mynah_launch3(d, kernel, gx, gy, nz, block, 0, stream, args);
     if (rc == 0) {
         uint32_t u32 = units, first = units / nz;   /* the units of split 0 */
         void *fargs[] = {&part, &res, &y, &r32, &t32, &first, &u32};
@@ -80,9 +132,11 @@ static int gemm_mfma_launch(mynah_device *d, int type, int ord, const void *w, s
     return rc;
 }
 
-static int gemm_mfma_on(void) {
+/* The MFMA kernels address a tile's 64 rows of x in 32 bits: longer rows take
+ * the VALU kernels. */
+static int gemm_mfma_on(size_t cols) {
     const char *env = getenv("MYNAH_GEMM_MFMA");
-    return env == NULL || env[0] != '0';
+    return (env == NULL || env[0] != '0') && cols < ((size_t)1 << 24);
 }
 
 int mynah_matmat_launch(mynah_device *d, int type, const void *w, size_t rows, size_t cols,
@@ -112,7 +166,7 @@ int mynah_matmat_launch(mynah_device *d, int type, const void *w, size_t rows, s
         mynah_set_error("misaligned operand for the batched GEMM");
         return -1;
     }
-    if (gemm_mfma_on())
+    if (gemm_mfma_on(cols))
         return gemm_mfma_launch(d, type, 0, w, rows, cols, rb, x, y, tokens, NULL, stream);
     const int k = type == MYNAH_Q4_K   ? MYNAH_K_Q4K_GEMM
                   : type == MYNAH_Q5_K ? MYNAH_K_Q5K_GEMM
@@ -147,7 +201,7 @@ int mynah_matmat_mv_launch(mynah_device *d, int type, const void *w, size_t rows
         mynah_set_error("misaligned operand for the matvec-order GEMM");
         return -1;
     }
-    if (gemm_mfma_on())
+    if (gemm_mfma_on(cols))
         return gemm_mfma_launch(d, type, 1, w, rows, cols, rb, x, y, tokens, res, stream);
     const int k = type == MYNAH_Q4_K   ? MYNAH_K_Q4K_GEMM_MV
                   : type == MYNAH_Q5_K ? MYNAH_K_Q5K_GEMM_MV
