@@ -19,7 +19,6 @@
 #include "runtime_internal.h"
 
 #include <pthread.h>
-#include <math.h>
 #include <stdlib.h>
 
 static int int8_mode = -1;
@@ -106,6 +105,44 @@ int mynah_q8_quantize_launch(mynah_device *d, const float *x, size_t tokens, siz
     return mynah_launch(d, MYNAH_K_Q8_QUANTIZE, (units + 3u) / 4u, 1, 256, 0, stream, args);
 }
 
+/* The batched kernels' workgroup tiles, in the kernel ids' order: how many fit
+ * a CU (LDS), and the microseconds one super-block takes with k of them there,
+ * t0 + k t1 (measured on MI355X at 512 and 2047 tokens; a lone small tile waits
+ * for its copies, full CUs issue). */
+typedef struct {
+    uint32_t rows, toks, waves, per_cu;
+    double t0, t1;
+} int8_tile;
+static const int8_tile int8_tiles[4] = {{32, 32, 4, 5, 1.1, 0.22},
+                                        {64, 64, 8, 2, 1.25, 0.7},
+                                        {96, 128, 16, 1, 0.0, 3.87},
+                                        {128, 128, 16, 1, 0.0, 4.9}};
+
+/* The tile of least estimated time: rounds of resident workgroups, the last
+ * with as many per CU as are left. The kernels address a tile's rows of
+ * weights and of activations in 32 bits: rows too long for the larger tiles
+ * take the smallest. MYNAH_INT8_TILE=0..3 forces one. */
+static int int8_plan(size_t rows, size_t tokens, size_t cols, uint32_t cus) {
+    const char *env = getenv("MYNAH_INT8_TILE");
+    if (env != NULL && env[0] >= '0' && env[0] <= '3' && env[1] == '\0') return env[0] - '0';
+    int best = 0;
+    double best_t = 0.0;
+    for (int i = 0; i < 4 && (i == 0 || cols < ((size_t)1 << 24)); i++) {
+        const int8_tile *t = &int8_tiles[i];
+        const uint64_t wgs = (uint64_t)((rows + t->rows - 1) / t->rows) *
+                             (uint64_t)((tokens + t->toks - 1) / t->toks);
+        const uint64_t slots = (uint64_t)cus * t->per_cu;
+        double us = (double)(wgs / slots) * (t->t0 + t->t1 * t->per_cu);
+        const uint64_t left = wgs % slots;
+        if (left) us += t->t0 + t->t1 * (double)((left + cus - 1) / cus);
+        if (i == 0 || us < best_t) {
+            best = i;
+            best_t = us;
+        }
+    }
+    return best;
+}
+
 int mynah_q4k_int8_launch(mynah_device *d, int type, const void *w, size_t rows, size_t cols,
                           const int8_t *xq, const float *xs, const int32_t *xsum, float *y,
                           size_t tokens, hipStream_t stream) {
@@ -132,42 +169,12 @@ int mynah_q4k_int8_launch(mynah_device *d, int type, const void *w, size_t rows,
     }
     uint32_t c32 = (uint32_t)cols, t32 = (uint32_t)tokens, tile = token_tile(cols);
     void *args[] = {&w, &xq, &xs, &xsum, &y, &r32, &c32, &t32, &nb, &tile};
-    /* Workgroup tile (32 tr) rows x (32 tt) tokens: the largest tile whose
-     * workgroups fill whole rounds of the chip (>= 90 % of the last round
-     * busy), given how many of each fit a CU (LDS: the double-buffered
-     * operands, 60 KiB for 2 x 2 down to 30 KiB for 1 x 1); else the tile
-     * with the fullest last round. */
-    static const int cand[4][3] = {{2, 2, 2}, {2, 1, 3}, {1, 2, 3}, {1, 1, 5}};
-    int tr = 1, tt = 1;
-    double best = -1.0;
-    for (int c = 0; c < 4; c++) {
-        const double wgs = (double)((rows + 32u * cand[c][0] - 1) / (32u * cand[c][0])) *
-                           (double)((tokens + 32u * cand[c][1] - 1) / (32u * cand[c][1]));
-        const double rounds = wgs / ((double)d->cus * cand[c][2]);
-        const double fill = rounds / ceil(rounds);
-        if (fill >= 0.9) {
-            tr = cand[c][0];
-            tt = cand[c][1];
-            break;
-        }
-        if (fill > best) {
-            best = fill;
-            tr = cand[c][0];
-            tt = cand[c][1];
-        }
-    }
-    const char *env = getenv("MYNAH_INT8_TILE");
-    if (env != NULL && env[0] >= '1' && env[0] <= '2' && env[1] >= '1' && env[1] <= '2') {
-        tr = env[0] - '0';
-        tt = env[1] - '0';
-    }
-    if (type == MYNAH_Q5_K) tr = tt = 2;      /* the one Q5_K tile */
-    const int k = type == MYNAH_Q5_K ? MYNAH_K_Q5K_GEMM_INT8_22
-                  : tr == 1 ? (tt == 1 ? MYNAH_K_Q4K_GEMM_INT8_11 : MYNAH_K_Q4K_GEMM_INT8_12)
-                            : (tt == 1 ? MYNAH_K_Q4K_GEMM_INT8_21 : MYNAH_K_Q4K_GEMM_INT8_22);
-    const size_t wr = (size_t)32 * tr, wt = (size_t)32 * tt;
-    return mynah_launch(d, k, (unsigned)((rows + wr - 1) / wr), (unsigned)((tokens + wt - 1) / wt),
-                        256, 0, stream, args);
+    const int8_tile *tl = &int8_tiles[int8_plan(rows, tokens, cols, (uint32_t)d->cus)];
+    const int k = (type == MYNAH_Q5_K ? MYNAH_K_Q5K_GEMM_INT8_32_32 : MYNAH_K_Q4K_GEMM_INT8_32_32) +
+                  (int)(tl - int8_tiles);
+    return mynah_launch(d, k, (unsigned)((rows + tl->rows - 1) / tl->rows),
+                        (unsigned)((tokens + tl->toks - 1) / tl->toks), 64u * tl->waves, 0,
+                        stream, args);
 }
 
 /* Workspace of one call: xq, xs, xsum, each 256-byte aligned. */

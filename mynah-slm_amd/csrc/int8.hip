@@ -166,327 +166,382 @@ extern "C" __global__ __launch_bounds__(256) void mynah_q4k_gemv_int8(
 }
 
 // ── batched int8 GEMM (tokens >= 2) ─────────────────────────────────────
-// A workgroup is 2 x 2 waves; wave (wr, wt) owns GI_TR 16-row tiles and GI_TT
-// 16-token tiles: rows R0 + 16 (GI_TR wr + i), tokens T0 + 16 (GI_TT wt + k).
+// A workgroup is WR x WT waves, each owning GI_TR 16-row tiles and GI_TT
+// 16-token tiles.
 // Per super-block and sub-block j, one v_mfma_i32_16x16x32_i8 per tile gives
-// the tile's integer dots: lane l feeds row (l % 16) of the tile with the 8
-// quants 8 (l / 16) .. +7 of the sub-block (A operand) and token (l % 16) with
-// the same 8 activation positions (B operand), and receives the dots of rows
-// 4 (l / 16) + e, e = 0..3, for token l % 16. Sub-blocks 2g and 2g+1 are the
-// low and high nibbles of the same 8 quant bytes: one 8-byte read per group.
+// the tile's integer dots, tokens as A and rows as B: lane l feeds token
+// (l % 16) and row (l % 16) with the 8 positions 8 (l / 16) .. + 7 of the
+// sub-block, and receives the dots of tokens 4 (l / 16) + e, e = 0..3, for row
+// l % 16. So a lane's scale and offset of a sub-block are one pair per row
+// tile, and its tokens' sums one float4 per token tile, shared by all its
+// tiles. Sub-blocks 2g and 2g+1 are the low and high nibbles of the same 8
+// quant bytes: one 8-byte read per group.
+// The accumulator starts at the bits of 1.5 * 2^23, whose unit is 1: the
+// integer result, read as a float, is 1.5 * 2^23 + dot (|dot| < 2^17), and one
+// subtraction gives the dot as an exact float. On gfx950 that subtraction (two
+// operands, a literal) issues at twice the rate of a conversion.
 // Operands go through LDS: per super-block the workgroup copies its rows'
-// quant bytes (Q5_K: qh and qs), its tokens' activations, sub-block sums and
-// scales straight from global memory into LDS (global_load_lds_dwordx4 /
-// _dword: no registers, nothing for the compiler to move), double buffered,
-// the next super-block's copy in flight while the current one is summed;
-// scale_j and offset_j of the rows are computed into LDS from the block
-// headers. One barrier per super-block. Quants and activations sit in LDS
-// chunk-major ([16-byte chunk][row or token][16 bytes]), so the 16 rows or
-// tokens one operand read spans are 16 bytes apart and every read of a
-// sub-block is the same per-lane address plus a constant. The dots of
-// sub-block j + 1 are issued before the epilogue of j.
+// quant bytes (Q5_K: qh and qs) and its tokens' activations and scales
+// straight from global memory into LDS (global_load_lds_dwordx4 / _dword: no
+// registers, nothing for the compiler to move), double buffered, the next
+// super-block's copy in flight while the current one is summed; the rows'
+// (scale_j, -offset_j) and the tokens' sums as floats are computed into LDS
+// from block headers and sums held in registers a super-block ahead. One
+// barrier per super-block.
+// What bounds it: issue. Per four tiles (1,024 outputs) and sub-block the four
+// i8 MFMAs (27 ns), 16 subtractions (18), 16 v_fmac (24) and the rank-one MFMA
+// (14) do not overlap on a SIMD: about 83 ns, where the form with a conversion
+// and both FMAs on the VALU took about 130. Measured on MI355X with the
+// quantiser, before (64 x 64 tiles, activations as the MFMA's columns) and now:
+// 9728 x 2560 Q4_K, 2047 tokens 347 -> 245 us; 6144 x 2048, 512 tokens 57 ->
+// 38 us; 4096 x 2560 Q5_K, 130 tokens 45 -> 28 us.
 // Q5_K (FMT 13, kernels.c:1155-1185 q5_k_quants): the same tiles, the quant
 // bytes at block offset 48 instead of 16, and each lane also holds the 8 qh
 // bytes of its 8 positions: bit j of qh[i] is the fifth bit (+16) of weight
 // i of sub-block j.
-// Bytes of one row's staged quant data per super-block: Q4_K qs (block bytes
-// 16 .. 143), Q5_K qh + qs (block bytes 16 .. 175).
-template <int FMT>
-constexpr uint32_t gi_qb() { return FMT == 13 ? 160u : 128u; }
-
 typedef __attribute__((address_space(3))) void gi_lds_void;
 
-// Copy super-block b of the workgroup's rows and tokens into LDS buffer
-// (lq, lx, lsum, lxs); wave w takes every fourth 64-chunk piece. Rows and
-// tokens past the ends read the last one (their results are not stored).
-// Copy super-block b of the workgroup's rows and tokens into LDS buffer
-// (lq, lx, lsum, lxs): lq[c][r] = 16-byte chunk c of row r's staged bytes,
-// lx[c][t] = chunk c of token t's 256 activations, lsum[t] = its 8 sums,
-// lxs[t] = its scale. Each copy instruction fills 1 KiB (64 lanes x 16
-// bytes); wave w takes every fourth one. Rows and tokens past the ends read
-// the last one (their results are not stored).
-template <int FMT, int GI_ROWS, int GI_TOK>
-MYNAH_DEV void gi_stage_async(uint8_t *lq, int8_t *lx, int32_t *lsum, float *lxs,
-                              const uint8_t *__restrict__ w, const int8_t *__restrict__ xq,
-                              const float *__restrict__ xs, const int32_t *__restrict__ xsum,
-                              uint32_t R0, uint32_t T0, uint32_t rows, uint32_t tokens,
-                              uint32_t cols, uint32_t nb, size_t rb, uint32_t b, uint32_t wave,
-                              uint32_t lane) {
-    constexpr uint32_t QB = gi_qb<FMT>(), CPR = QB / 16u, UB = FMT == 13 ? 176u : 144u;
-    constexpr uint32_t NQ = GI_ROWS * CPR / 64u, NX = GI_TOK * 16u / 64u, NS = GI_TOK * 2u / 64u;
-    // Workgroup-uniform bases; per-lane offsets stay below 4 GiB (at most 64
-    // rows or tokens of the tile).
-    const uint8_t *wb = w + (size_t)R0 * rb + (size_t)b * UB + 16u;
-    const int8_t *xb = xq + (size_t)T0 * cols + 256u * b;
-    const int32_t *sb = xsum + ((size_t)T0 * nb + b) * 8u;
-    const uint32_t rmax = rows - 1u - R0, tmax = tokens - 1u - T0;
-#pragma unroll
-    for (uint32_t k = 0; k < (NQ + 3u) / 4u; k++) {
-        const uint32_t n = 4u * k + wave;
-        if (n < NQ) {
-            const uint32_t p = 64u * n + lane, c = p / GI_ROWS, r = p - c * GI_ROWS;
-            const uint32_t rr = r < rmax ? r : rmax;
-            __builtin_amdgcn_global_load_lds((const void *)(wb + (uint32_t)(rr * (uint32_t)rb +
-                                                                              16u * c)),
-                                             (gi_lds_void *)(lq + 1024u * n), 16, 0, 0);
-        }
-    }
-#pragma unroll
-    for (uint32_t k = 0; k < (NX + 3u) / 4u; k++) {
-        const uint32_t n = 4u * k + wave;
-        if (n < NX) {
-            const uint32_t p = 64u * n + lane, c = p / GI_TOK, t = p - c * GI_TOK;
-            const uint32_t tt = t < tmax ? t : tmax;
-            __builtin_amdgcn_global_load_lds((const void *)(xb + (uint32_t)(tt * cols + 16u * c)),
-                                             (gi_lds_void *)(lx + 1024u * n), 16, 0, 0);
-        }
-    }
-#pragma unroll
-    for (uint32_t k = 0; k < (NS + 3u) / 4u; k++) {
-        const uint32_t n = 4u * k + wave;
-        if (n < NS) {
-            const uint32_t p = 64u * n + lane, t = p >> 1, tt = t < tmax ? t : tmax;
-            __builtin_amdgcn_global_load_lds(
-                (const void *)(sb + (uint32_t)(tt * nb * 8u + 4u * (p & 1u))),
-                (gi_lds_void *)(lsum + 256u * n), 16, 0, 0);
-        }
-    }
-    if (wave == 3u && lane < (uint32_t)GI_TOK) {
-        const uint32_t tt = lane < tmax ? lane : tmax;
-        __builtin_amdgcn_global_load_lds((const void *)(xs + (size_t)T0 * nb + b + tt * nb),
-                                         (gi_lds_void *)lxs, 4, 0, 0);
-    }
-}
+// One super-block's operands in LDS. A row's 128 quant bytes and a token's 256
+// activations lie contiguous, 16-byte chunk c at place c ^ (row / 2 % 8) or c ^
+// (token % 16), so that both the copies' global reads (whole rows) and the
+// operand reads (16 rows or tokens, one chunk) meet no conflict.
+template <int FMT, int ROWS, int TOK> struct GiBuf {
+    uint8_t q[ROWS * 128];
+    int8_t x[TOK * 256];
+    uint8_t qh[FMT == 13 ? ROWS * 32 : 16];
+    float sc[8 * ROWS];              // scale_j of row r at ROWS j + r
+    float no[8 * ROWS];              // -offset_j
+    float fsum[8 * TOK];             // sum_j of token t at TOK j + t
+    float xs[TOK];
+};
 
-// Scale and offset of sub-blocks hj, hj + 1 of the staged row, into LDS.
-template <int GI_ROWS>
-MYNAH_DEV void gi_stage(float *buf, const uint4 hdr, uint32_t hj, uint32_t row) {
+// The copies of a workgroup of NW waves: instruction n (1 KiB: 64 lanes x 16
+// bytes) is wave n % NW's; per lane its byte offset from the tile's first row
+// or token, the super-block a scalar offset. Rows and tokens past the ends
+// read the last one (their results are not stored).
+template <int FMT, int ROWS, int TOK, int NW> struct GiCopy {
+    static constexpr int NQ = ROWS / 8, NX = TOK / 4, NH = FMT == 13 ? ROWS / 32 : 0;
+    static constexpr int PQ = (NQ + NW - 1) / NW, PX = (NX + NW - 1) / NW;
+    uint32_t qo[PQ], xo[PX], ho, so;
+    __amdgpu_buffer_rsrc_t rq, rx, rs;
+    __device__ __forceinline__ void init(const uint8_t *w, const int8_t *xq, const float *xs,
+                                         uint32_t R0, uint32_t T0, uint32_t rows, uint32_t tokens,
+                                         uint32_t cols, uint32_t nb, uint32_t rb, uint32_t wave,
+                                         uint32_t lane) {
+        const uint32_t rmax = rows - 1u - R0, tmax = tokens - 1u - T0;
+#pragma unroll
+        for (int k = 0; k < PQ; k++) {
+            const uint32_t r = 8u * (NW * k + wave) + (lane >> 3), p = lane & 7u;
+            qo[k] = (r < rmax ? r : rmax) * rb + 16u * (p ^ ((r >> 1) & 7u)) +
+                    (FMT == 13 ? 48u : 16u);
+        }
+#pragma unroll
+        for (int k = 0; k < PX; k++) {
+            const uint32_t t = 4u * (NW * k + wave) + (lane >> 4), p = lane & 15u;
+            xo[k] = (t < tmax ? t : tmax) * cols + 16u * (p ^ (t & 15u));
+        }
+        const uint32_t hr = 32u * wave + (lane >> 1), st = 64u * wave + lane;
+        ho = (hr < rmax ? hr : rmax) * rb + 16u * (lane & 1u) + 16u;
+        so = (st < tmax ? st : tmax) * nb * 4u;
+        rq = __builtin_amdgcn_make_buffer_rsrc((void *)(w + (size_t)R0 * rb), 0, 0xffffffffu,
+                                               0x00020000);
+        rx = __builtin_amdgcn_make_buffer_rsrc((void *)(xq + (size_t)T0 * cols), 0, 0xffffffffu,
+                                               0x00020000);
+        rs = __builtin_amdgcn_make_buffer_rsrc((void *)(xs + (size_t)T0 * nb), 0, 0xffffffffu,
+                                               0x00020000);
+    }
+    __device__ __forceinline__ void copy(GiBuf<FMT, ROWS, TOK> &buf, uint32_t b,
+                                         uint32_t wave) const {
+        constexpr uint32_t UB = FMT == 13 ? 176u : 144u;
+#pragma unroll
+        for (int k = 0; k < PQ; k++)
+            if (NW * k + wave < (uint32_t)NQ)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    rq, (gi_lds_void *)(buf.q + 1024u * (NW * k + wave)), 16, qo[k], UB * b, 0, 0);
+#pragma unroll
+        for (int k = 0; k < PX; k++)
+            if (NW * k + wave < (uint32_t)NX)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    rx, (gi_lds_void *)(buf.x + 1024u * (NW * k + wave)), 16, xo[k], 256u * b, 0,
+                    0);
+        if (FMT == 13 && wave < (uint32_t)NH)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                rq, (gi_lds_void *)(buf.qh + 1024u * wave), 16, ho, UB * b, 0, 0);
+        if (64u * wave < (uint32_t)TOK) {
+            if (TOK % 64 == 0 || (threadIdx.x & 63u) < (uint32_t)TOK)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    rs, (gi_lds_void *)(buf.xs + 64u * wave), 4, so, 4u * b, 0, 0);
+        }
+    }
+};
+
+// Scale and -offset of sub-blocks hj, hj + 1 of the staged row, into LDS.
+template <int ROWS>
+MYNAH_DEV void gi_stage(float *sc, float *no, const uint4 hdr, uint32_t hj, uint32_t row) {
 #pragma clang fp contract(off)
     const float d = f16_to_f32(hdr.x), dmin = f16_to_f32(hdr.x >> 16);
-    uint32_t s0, m0, s1, m1;
-    q4k_scale_min(hdr.y, hdr.z, hdr.w, hj, &s0, &m0);
-    q4k_scale_min(hdr.y, hdr.z, hdr.w, hj + 1u, &s1, &m1);
-    buf[hj * GI_ROWS + row] = d * (float)s0;
-    buf[(hj + 1u) * GI_ROWS + row] = d * (float)s1;
-    buf[(8u + hj) * GI_ROWS + row] = dmin * (float)m0;
-    buf[(9u + hj) * GI_ROWS + row] = dmin * (float)m1;
+    float s0, m0, s1, m1;
+    q4k_sm_rt(hdr.y, hdr.z, hdr.w, hj, s0, m0);
+    q4k_sm_rt(hdr.y, hdr.z, hdr.w, hj + 1u, s1, m1);
+    sc[hj * ROWS + row] = d * s0;
+    sc[(hj + 1u) * ROWS + row] = d * s1;
+    no[hj * ROWS + row] = -(dmin * m0);
+    no[(hj + 1u) * ROWS + row] = -(dmin * m1);
 }
 
-// One super-block's dots and epilogue from the LDS buffers: lane l's rows
-// 16 (GI_TR wr + i) + l % 16 and tokens 16 (GI_TT wt + k) + l % 16, quant and
-// activation positions 32 g + 8 (l / 16) .. +7 of group g / sub-block j;
-// tot[i][k][e] over j = 0..7 in order, then acc += tot * xs. MIXED: some
-// lane has a token outside the groups of four, which takes the plain form.
-template <int FMT, bool MIXED, int GI_TR, int GI_TT>
-MYNAH_DEV void gi_block(float (&acc)[GI_TR][GI_TT][4], const uint8_t *lq, const int8_t *lx,
-                        const int32_t *lsum, const float *lxs, const float4 *sbuf, uint32_t wr,
-                        uint32_t wt, uint32_t lane, const bool (&fma_path)[GI_TT]) {
+// Four of a token's eight sums as floats (exact: |sum| <= 32 * 127), into LDS
+// by sub-block.
+template <int TOK>
+MYNAH_DEV void gi_stage_sums(float *fsum, const int4 v, uint32_t half, uint32_t tok) {
+    float *p = fsum + 4u * half * TOK + tok;
+    p[0] = (float)v.x;
+    p[TOK] = (float)v.y;
+    p[2 * TOK] = (float)v.z;
+    p[3 * TOK] = (float)v.w;
+}
+
+// The bits of 1.5 * 2^23.
+#define GI_MAGIC 0x4b400000
+
+typedef float gi_f32x16 __attribute__((ext_vector_type(16)));
+
+// One super-block's dots and epilogue from the LDS buffer, for the wave whose
+// rows start at r0 and tokens at t0 of the tile. Tile n = GI_TT i + k of the
+// wave is rows 16 i .. + 15, tokens 16 k .. + 15; lane l holds of it row l % 16
+// and tokens 4 (l / 16) + e, in element 4 (n % 4) + e of tot[n / 4]. Over j =
+// 0..7 in order tot = fma(xsum_j, -offset_j, fma(dot_j, scale_j, tot)), then
+// acc += tot * xs. The second fma of four tiles is one MFMA: the outer product
+// of 16 sums and 16 offsets per block, accumulated with fmaf's one rounding
+// (13.7 ns against 16 v_fmac's 23.5); tiles past the last whole four take
+// v_fmac. MIXED: some lane has a token outside the groups of four, which takes
+// the plain form total += scale * dot - offset * sum (fma_path bit 4 k + e: the
+// token's groups-of-four form).
+template <int FMT, bool MIXED, int GI_TR, int GI_TT, int ROWS, int TOK>
+MYNAH_DEV void gi_block(gi_f32x16 (&acc)[(GI_TR * GI_TT + 3) / 4],
+                        const GiBuf<FMT, ROWS, TOK> &buf, uint32_t r0, uint32_t t0,
+                        uint32_t lane, uint32_t fma_path) {
 #pragma clang fp contract(off)
-    constexpr int GI_ROWS = 32 * GI_TR, GI_TOK = 32 * GI_TT;
+    constexpr int NT = GI_TR * GI_TT, NG = (NT + 3) / 4, NM = MIXED ? 0 : NT / 4;
     const uint32_t lm = lane & 15u, lk = lane >> 4;
     // Lane l reads the 8 bytes at position 8 (l / 16) of a 32-byte group:
     // chunk 2 g + (l / 16) / 2 of its row / token, half (l / 16) % 2.
-    const uint32_t lo = 16u * (lk >> 1), hb = 8u * (lk & 1u);
-    const uint8_t *qrow[GI_TR];
-    const int8_t *xrow[GI_TT];
-    uint32_t tl[GI_TT];
+    const uint32_t ck = lk >> 1, hb = 8u * (lk & 1u), sq = lm >> 1, sx = lm;
+    const uint8_t *qrow = buf.q + 128u * (r0 + lm) + hb;
+    const int8_t *xrow = buf.x + 256u * (t0 + lm) + hb;
+    const float *srow = buf.sc + r0 + lm, *nrow = buf.no + r0 + lm;
+    const float *frow = buf.fsum + t0 + 4u * lk;
+    // Operands of the rank-one MFMA m: lane l feeds its block l / 16's tile.
+    const float *mf[NM > 0 ? NM : 1], *mn[NM > 0 ? NM : 1];
 #pragma unroll
-    for (int i = 0; i < GI_TR; i++)
-        qrow[i] = lq + 16u * (16u * (GI_TR * wr + (uint32_t)i) + lm) + hb + lo * GI_ROWS;
-#pragma unroll
-    for (int k = 0; k < GI_TT; k++) {
-        tl[k] = 16u * (GI_TT * wt + (uint32_t)k) + lm;
-        xrow[k] = lx + 16u * tl[k] + hb + lo * GI_TOK;
+    for (int m = 0; m < NM; m++) {
+        const uint32_t n = 4u * m + lk;
+        mf[m] = buf.fsum + t0 + 16u * (n % GI_TT) + lm;
+        mn[m] = buf.no + r0 + 16u * (n / GI_TT) + lm;
     }
-    unsigned long long qh[GI_TR];
+    uint2 qh[GI_TR];
     if (FMT == 13) {
 #pragma unroll
-        for (int i = 0; i < GI_TR; i++) qh[i] = *(const unsigned long long *)qrow[i];
+        for (int i = 0; i < GI_TR; i++)
+            qh[i] = *(const uint2 *)(buf.qh + 32u * (r0 + lm + 16u * i) + 8u * lk);
     }
-    // Dots of sub-block j: the quant bytes of group j / 2 of each row tile
-    // (Q5_K: its qs start at chunk 2), nibble j % 2, times the activations
-    // of sub-block j of each token tile. The loop below stays rolled (runtime
-    // j), so no more than two sub-blocks' dots are ever live.
-    auto dots = [&](i32x4 (&dt)[GI_TR][GI_TT], uint32_t j) {
-        unsigned long long xb[GI_TT];
+    const i32x4 magic = {GI_MAGIC, GI_MAGIC, GI_MAGIC, GI_MAGIC};
+    const gi_f32x16 zero = {};
+    gi_f32x16 tot[NG];
 #pragma unroll
-        for (int k = 0; k < GI_TT; k++)
-            xb[k] = *(const unsigned long long *)(xrow[k] + 16u * GI_TOK * 2u * j);
+    for (int m = 0; m < NG; m++) tot[m] = zero;
+    // Two sub-blocks (a group of quant bytes) per round of the loop, which
+    // stays rolled, so no more than one group's dots are ever live.
+#pragma unroll 1
+    for (uint32_t g = 0; g < 4u; g++) {
+        uint2 qa[GI_TR];
 #pragma unroll
-        for (int i = 0; i < GI_TR; i++) {
-            const uint32_t c = (FMT == 13 ? 2u : 0u) + 2u * (j >> 1);
-            const unsigned long long qa =
-                *(const unsigned long long *)(qrow[i] + 16u * GI_ROWS * c);
-            unsigned long long q = (qa >> (4u * (j & 1u))) & 0x0f0f0f0f0f0f0f0full;
-            if (FMT == 13) q |= ((qh[i] >> j) & 0x0101010101010101ull) << 4;
+        for (int i = 0; i < GI_TR; i++)
+            qa[i] = *(const uint2 *)(qrow + 2048u * i + 16u * ((2u * g + ck) ^ sq));
+        i32x4 dt[2][NT];
 #pragma unroll
-            for (int k = 0; k < GI_TT; k++) {
-                const i32x4 zero = {0, 0, 0, 0};
-                dt[i][k] = __builtin_amdgcn_mfma_i32_16x16x32_i8((long)q, (long)xb[k], zero, 0, 0,
-                                                                 0);
+        for (int h = 0; h < 2; h++) {
+            long xb[GI_TT];
+#pragma unroll
+            for (int k = 0; k < GI_TT; k++)
+                xb[k] = *(const long *)(xrow + 4096u * k + 16u * ((4u * g + 2u * h + ck) ^ sx));
+#pragma unroll
+            for (int i = 0; i < GI_TR; i++) {
+                uint2 v = qa[i];
+                if (h) v = make_uint2(v.x >> 4, v.y >> 4);
+                v = make_uint2(v.x & 0x0f0f0f0fu, v.y & 0x0f0f0f0fu);
+                if (FMT == 13) {
+                    const uint32_t j = 2u * g + h;
+                    v.x |= ((qh[i].x >> j) & 0x01010101u) << 4;
+                    v.y |= ((qh[i].y >> j) & 0x01010101u) << 4;
+                }
+                const long q = (long)(((unsigned long long)v.y << 32) | v.x);
+#pragma unroll
+                for (int k = 0; k < GI_TT; k++)
+                    dt[h][GI_TT * i + k] =
+                        __builtin_amdgcn_mfma_i32_16x16x32_i8(xb[k], q, magic, 0, 0, 0);
             }
         }
-    };
-    float tot[GI_TR][GI_TT][4];
 #pragma unroll
-    for (int i = 0; i < GI_TR; i++)
+        for (int h = 0; h < 2; h++) {
+            const uint32_t j = 2u * g + h;
+            float sc[GI_TR], no[GI_TR];
+            float4 fs[GI_TT];
 #pragma unroll
-        for (int k = 0; k < GI_TT; k++)
+            for (int i = 0; i < GI_TR; i++) {
+                sc[i] = srow[j * ROWS + 16u * i];
+                if (GI_TT * (i + 1) > 4 * NM) no[i] = nrow[j * ROWS + 16u * i];
+            }
+            if (NT > 4 * NM) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) tot[i][k][e] = 0.0f;
-    // tot = fma(-xsum_j, offset_j, fma(dot_j, scale_j, tot)) for sub-block j.
-    auto epi = [&](const i32x4 (&dt)[GI_TR][GI_TT], uint32_t j) {
-        float xsj[GI_TT];
+                for (int k = 0; k < GI_TT; k++)
+                    fs[k] = *(const float4 *)(frow + j * TOK + 16u * k);
+            }
 #pragma unroll
-        for (int k = 0; k < GI_TT; k++) xsj[k] = (float)lsum[8u * tl[k] + j];
-#pragma unroll
-        for (int i = 0; i < GI_TR; i++) {
-            const uint32_t slot = (16u * (GI_TR * wr + i)) / 4u + lk;
-            const float4 sc = sbuf[j * (GI_ROWS / 4) + slot];
-            const float4 of = sbuf[(8u + j) * (GI_ROWS / 4) + slot];
-            const float scv[4] = {sc.x, sc.y, sc.z, sc.w};
-            const float ofv[4] = {of.x, of.y, of.z, of.w};
-#pragma unroll
-            for (int k = 0; k < GI_TT; k++) {
+            for (int n = 0; n < NT; n++) {
+                const int i = n / GI_TT, k = n % GI_TT;
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                    const float dv = (float)dt[i][k][e];
-                    float f = __builtin_fmaf(dv, scv[e], tot[i][k][e]);
-                    f = __builtin_fmaf(-xsj[k], ofv[e], f);
-                    if (MIXED) {
-                        const float p = tot[i][k][e] + (scv[e] * dv - ofv[e] * xsj[k]);
-                        f = fma_path[k] ? f : p;
+                    const float dv = __int_as_float(dt[h][n][e]) - 12582912.0f;
+                    const float t = tot[n / 4][4 * (n % 4) + e];
+                    float f = __builtin_fmaf(dv, sc[i], t);
+                    if (n >= 4 * NM) {
+                        const float xsv = e == 0   ? fs[k].x
+                                          : e == 1 ? fs[k].y
+                                          : e == 2 ? fs[k].z
+                                                   : fs[k].w;
+                        f = __builtin_fmaf(xsv, no[i], f);
+                        if (MIXED) {
+                            const float p = t + (sc[i] * dv + no[i] * xsv);
+                            f = (fma_path >> (4 * k + e)) & 1u ? f : p;
+                        }
                     }
-                    tot[i][k][e] = f;
+                    tot[n / 4][4 * (n % 4) + e] = f;
                 }
             }
+#pragma unroll
+            for (int m = 0; m < NM; m++)
+                tot[m] = __builtin_amdgcn_mfma_f32_16x16x1f32(mf[m][j * TOK], mn[m][j * ROWS],
+                                                              tot[m], 0, 0, 0);
         }
-    };
-    // Two register sets of dots, alternating: the dots of sub-block j + 1
-    // are issued before the epilogue of j, with no copies between them.
-    i32x4 da[GI_TR][GI_TT], db[GI_TR][GI_TT];
-    dots(da, 0u);
-#pragma unroll 1
-    for (uint32_t j = 0; j < 6u; j += 2u) {
-        dots(db, j + 1u);
-        epi(da, j);
-        dots(da, j + 2u);
-        epi(db, j + 1u);
     }
-    dots(db, 7u);
-    epi(da, 6u);
-    epi(db, 7u);
 #pragma unroll
-    for (int i = 0; i < GI_TR; i++)
+    for (int n = 0; n < NT; n++) {
+        const float4 x4 = *(const float4 *)(buf.xs + t0 + 16u * (n % GI_TT) + 4u * lk);
+        const float xsv[4] = {x4.x, x4.y, x4.z, x4.w};
 #pragma unroll
-        for (int k = 0; k < GI_TT; k++) {
-            const float xsv = lxs[tl[k]];
-#pragma unroll
-            for (int e = 0; e < 4; e++) acc[i][k][e] = acc[i][k][e] + tot[i][k][e] * xsv;
-        }
+        for (int e = 0; e < 4; e++)
+            acc[n / 4][4 * (n % 4) + e] =
+                acc[n / 4][4 * (n % 4) + e] + tot[n / 4][4 * (n % 4) + e] * xsv[e];
+    }
 }
 
-template <int FMT, int GI_TR, int GI_TT>
+// WR x WT waves; ROWS = 16 GI_TR WR, TOK = 16 GI_TT WT.
+template <int FMT, int WR, int WT, int GI_TR, int GI_TT>
 MYNAH_DEV void gemm_int8(const uint8_t *__restrict__ w, const int8_t *__restrict__ xq,
                          const float *__restrict__ xs, const int32_t *__restrict__ xsum,
                          float *__restrict__ y, uint32_t rows, uint32_t cols, uint32_t tokens,
                          uint32_t nb, uint32_t tile) {
-    constexpr int GI_ROWS = 32 * GI_TR, GI_TOK = 32 * GI_TT;
-    constexpr uint32_t QB = gi_qb<FMT>();
-    __shared__ __attribute__((aligned(16))) uint8_t lq[2][GI_ROWS * QB];
-    __shared__ __attribute__((aligned(16))) int8_t lx[2][GI_TOK * 256];
-    __shared__ __attribute__((aligned(16))) int32_t lsum[2][GI_TOK * 8];
-    __shared__ __attribute__((aligned(16))) float lxs[2][GI_TOK];
-    __shared__ float4 so[2][16 * GI_ROWS / 4];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const uint32_t wr = wave & 1u, wt = wave >> 1;
-    const uint32_t R0 = blockIdx.x * GI_ROWS, T0 = blockIdx.y * GI_TOK;
-    const size_t rb = (size_t)nb * (FMT == 13 ? 176u : 144u);
+    constexpr int ROWS = 16 * GI_TR * WR, TOK = 16 * GI_TT * WT, NW = WR * WT;
+    static_assert(4 * ROWS <= 64 * NW && 2 * TOK <= 64 * NW && ROWS % 32 == 0 && TOK % 4 == 0,
+                  "staging roles");
+    constexpr uint32_t UB = FMT == 13 ? 176u : 144u;
+    __shared__ __attribute__((aligned(16))) GiBuf<FMT, ROWS, TOK> buf[2];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t r0 = 16u * GI_TR * (wave % WR), t0 = 16u * GI_TT * (wave / WR);
+    const uint32_t R0 = blockIdx.x * ROWS, T0 = blockIdx.y * TOK;
+    const uint32_t rb = nb * UB;
     const uint32_t lm = lane & 15u, lk = lane >> 4;
 
-    uint32_t tok[GI_TT];
-    bool fma_path[GI_TT];
-    bool all_fma = true;
+    // Bit 4 k + e: token T0 + t0 + 16 k + 4 lk + e falls in a whole group of
+    // four of its token tile.
+    uint32_t fma_path = 0u;
 #pragma unroll
-    for (int k = 0; k < GI_TT; k++) {
-        const uint32_t t = T0 + 16u * (GI_TT * wt + k) + lm;
-        tok[k] = t;
-        const uint32_t tc = t < tokens ? t : tokens - 1u;
-        const uint32_t t0 = tc - tc % tile;
-        const uint32_t cnt = tokens - t0 < tile ? tokens - t0 : tile;
-        fma_path[k] = tc - t0 < (cnt & ~3u);
-        all_fma = all_fma && fma_path[k];
-    }
-    const bool mixed = !__all(all_fma);
+    for (uint32_t k = 0; k < GI_TT; k++)
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; e++) {
+            const uint32_t t = T0 + t0 + 16u * k + 4u * lk + e;
+            const uint32_t tc = t < tokens ? t : tokens - 1u;
+            const uint32_t tb = tc - tc % tile;
+            const uint32_t cnt = tokens - tb < tile ? tokens - tb : tile;
+            fma_path |= (tc - tb < (cnt & ~3u) ? 1u : 0u) << (4u * k + e);
+        }
+    const bool mixed = !__all(fma_path == (1u << (4 * GI_TT)) - 1u);
     // Scale staging: thread tid owns row tid / 4 of the workgroup, sub-blocks
-    // 2 (tid % 4) and 2 (tid % 4) + 1 (threads beyond 4 GI_ROWS stage nothing).
+    // 2 (tid % 4) and 2 (tid % 4) + 1; sum staging: token tid / 2, sub-blocks
+    // 4 (tid % 2) .. + 3 (threads beyond stage none).
     const uint32_t srow = tid >> 2, hj = 2u * (tid & 3u);
-    const bool stager = srow < GI_ROWS;
-    uint32_t hr = R0 + (stager ? srow : 0u);
+    const bool stager = srow < ROWS, summer = tid < 2u * TOK;
+    uint32_t hr = R0 + (stager ? srow : 0u), st = T0 + (summer ? tid >> 1 : 0u);
     hr = hr < rows ? hr : rows - 1u;
+    st = st < tokens ? st : tokens - 1u;
     const uint8_t *hrow = w + (size_t)hr * rb;
-    constexpr uint32_t UB = FMT == 13 ? 176u : 144u;
+    const int4 *sumrow = (const int4 *)(xsum + (size_t)st * nb * 8u) + (tid & 1u);
 
-    float acc[GI_TR][GI_TT][4];
+    constexpr int NG = (GI_TR * GI_TT + 3) / 4;
+    const gi_f32x16 zero = {};
+    gi_f32x16 acc[NG];
 #pragma unroll
-    for (int i = 0; i < GI_TR; i++)
-#pragma unroll
-        for (int k = 0; k < GI_TT; k++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) acc[i][k][e] = 0.0f;
+    for (int m = 0; m < NG; m++) acc[m] = zero;
 
-    gi_stage_async<FMT, GI_ROWS, GI_TOK>(lq[0], lx[0], lsum[0], lxs[0], w, xq, xs, xsum, R0, T0,
-                                         rows, tokens, cols, nb, rb, 0u, wave, lane);
+    GiCopy<FMT, ROWS, TOK, NW> cp;
+    cp.init(w, xq, xs, R0, T0, rows, tokens, cols, nb, rb, wave, lane);
+    cp.copy(buf[0], 0u, wave);
     uint4 hdr = *(const uint4 *)hrow;
+    int4 sums = sumrow[0];
     __builtin_amdgcn_s_waitcnt(0);
-    if (stager) gi_stage<GI_ROWS>((float *)so[0], hdr, hj, srow);
+    if (stager) gi_stage<ROWS>(buf[0].sc, buf[0].no, hdr, hj, srow);
+    if (summer) gi_stage_sums<TOK>(buf[0].fsum, sums, tid & 1u, tid >> 1);
     __syncthreads();
     for (uint32_t b = 0; b < nb; b++) {
         const uint32_t c = b & 1u;
         const bool more = b + 1u < nb;
         if (more) {
-            gi_stage_async<FMT, GI_ROWS, GI_TOK>(lq[c ^ 1u], lx[c ^ 1u], lsum[c ^ 1u],
-                                                 lxs[c ^ 1u], w, xq, xs, xsum, R0, T0, rows,
-                                                 tokens, cols, nb, rb, b + 1u, wave, lane);
             hdr = *(const uint4 *)(hrow + (size_t)(b + 1u) * UB);
+            sums = sumrow[2u * (b + 1u)];
+            cp.copy(buf[c ^ 1u], b + 1u, wave);
         }
         if (mixed)
-            gi_block<FMT, true>(acc, lq[c], lx[c], lsum[c], lxs[c], so[c], wr, wt, lane,
-                                fma_path);
+            gi_block<FMT, true, GI_TR, GI_TT, ROWS, TOK>(acc, buf[c], r0, t0, lane, fma_path);
         else
-            gi_block<FMT, false>(acc, lq[c], lx[c], lsum[c], lxs[c], so[c], wr, wt, lane,
-                                 fma_path);
+            gi_block<FMT, false, GI_TR, GI_TT, ROWS, TOK>(acc, buf[c], r0, t0, lane, fma_path);
         if (more) {
             __builtin_amdgcn_s_waitcnt(0);
-            if (stager) gi_stage<GI_ROWS>((float *)so[c ^ 1u], hdr, hj, srow);
+            if (stager) gi_stage<ROWS>(buf[c ^ 1u].sc, buf[c ^ 1u].no, hdr, hj, srow);
+            if (summer) gi_stage_sums<TOK>(buf[c ^ 1u].fsum, sums, tid & 1u, tid >> 1);
         }
         __syncthreads();
     }
 
 #pragma unroll
-    for (int i = 0; i < GI_TR; i++)
+    for (int k = 0; k < GI_TT; k++)
 #pragma unroll
-        for (int k = 0; k < GI_TT; k++) {
-            if (tok[k] >= tokens) continue;
-            float *yo = y + (size_t)tok[k] * rows;
+        for (uint32_t e = 0; e < 4u; e++) {
+            const uint32_t t = T0 + t0 + 16u * k + 4u * lk + e;
+            if (t >= tokens) continue;
+            float *yo = y + (size_t)t * rows;
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const uint32_t r = R0 + 16u * (GI_TR * wr + i) + 4u * lk + e;
-                if (r < rows) yo[r] = acc[i][k][e];
+            for (int i = 0; i < GI_TR; i++) {
+                const uint32_t r = R0 + r0 + 16u * i + lm;
+                if (r < rows) yo[r] = acc[(GI_TT * i + k) / 4][4 * ((GI_TT * i + k) % 4) + e];
             }
         }
 }
 
-#define GEMM_INT8(NAME, FMT, TR, TT)                                                         \
-    extern "C" __global__ __launch_bounds__(256, 2) void NAME##_##TR##TT(                    \
-        const uint8_t *__restrict__ w, const int8_t *__restrict__ xq,                        \
-        const float *__restrict__ xs, const int32_t *__restrict__ xsum,                      \
-        float *__restrict__ y, uint32_t rows, uint32_t cols, uint32_t tokens, uint32_t nb,   \
-        uint32_t tile) {                                                                     \
-        gemm_int8<FMT, TR, TT>(w, xq, xs, xsum, y, rows, cols, tokens, nb, tile);            \
+// ROWSxTOK: the workgroup's tile, of 16 waves (four per SIMD) where it is
+// large. The tiles the host chooses among, by rows and tokens (int8.c).
+#define GEMM_INT8(NAME, FMT, WR, WT, TR, TT, TILE)                                           \
+    extern "C" __global__ __launch_bounds__(64 * WR * WT, WR * WT == 16 ? 4 : 2) void        \
+        NAME##_##TILE(const uint8_t *__restrict__ w, const int8_t *__restrict__ xq,          \
+                      const float *__restrict__ xs, const int32_t *__restrict__ xsum,        \
+                      float *__restrict__ y, uint32_t rows, uint32_t cols, uint32_t tokens,  \
+                      uint32_t nb, uint32_t tile) {                                          \
+        gemm_int8<FMT, WR, WT, TR, TT>(w, xq, xs, xsum, y, rows, cols, tokens, nb, tile);    \
     }
-GEMM_INT8(mynah_q4k_gemm_int8, 12, 1, 1)
-GEMM_INT8(mynah_q4k_gemm_int8, 12, 1, 2)
-GEMM_INT8(mynah_q4k_gemm_int8, 12, 2, 1)
-GEMM_INT8(mynah_q4k_gemm_int8, 12, 2, 2)
-GEMM_INT8(mynah_q5k_gemm_int8, 13, 2, 2)
+#define GEMM_INT8_TILES(NAME, FMT)                                                           \
+    GEMM_INT8(NAME, FMT, 2, 2, 1, 1, 32x32)                                                  \
+    GEMM_INT8(NAME, FMT, 4, 2, 1, 2, 64x64)                                                  \
+    GEMM_INT8(NAME, FMT, 2, 8, 3, 1, 96x128)                                                 \
+    GEMM_INT8(NAME, FMT, 4, 4, 2, 2, 128x128)
+GEMM_INT8_TILES(mynah_q4k_gemm_int8, 12)
+GEMM_INT8_TILES(mynah_q5k_gemm_int8, 13)

@@ -94,11 +94,14 @@ enum { MYNAH_Q4_0 = 2, MYNAH_Q8_0 = 8, MYNAH_Q4_K = 12, MYNAH_Q5_K = 13, MYNAH_Q
     X(MYNAH_K_EXPF, "mynah_expf_map")                  \
     X(MYNAH_K_Q8_QUANTIZE, "mynah_q8_quantize")        \
     X(MYNAH_K_Q4K_GEMV_INT8, "mynah_q4k_gemv_int8")    \
-    X(MYNAH_K_Q4K_GEMM_INT8_11, "mynah_q4k_gemm_int8_11") \
-    X(MYNAH_K_Q4K_GEMM_INT8_12, "mynah_q4k_gemm_int8_12") \
-    X(MYNAH_K_Q4K_GEMM_INT8_21, "mynah_q4k_gemm_int8_21") \
-    X(MYNAH_K_Q4K_GEMM_INT8_22, "mynah_q4k_gemm_int8_22") \
-    X(MYNAH_K_Q5K_GEMM_INT8_22, "mynah_q5k_gemm_int8_22")
+    X(MYNAH_K_Q4K_GEMM_INT8_32_32, "mynah_q4k_gemm_int8_32x32") \
+    X(MYNAH_K_Q4K_GEMM_INT8_64_64, "mynah_q4k_gemm_int8_64x64") \
+    X(MYNAH_K_Q4K_GEMM_INT8_96_128, "mynah_q4k_gemm_int8_96x128") \
+    X(MYNAH_K_Q4K_GEMM_INT8_128_128, "mynah_q4k_gemm_int8_128x128") \
+    X(MYNAH_K_Q5K_GEMM_INT8_32_32, "mynah_q5k_gemm_int8_32x32") \
+    X(MYNAH_K_Q5K_GEMM_INT8_64_64, "mynah_q5k_gemm_int8_64x64") \
+    X(MYNAH_K_Q5K_GEMM_INT8_96_128, "mynah_q5k_gemm_int8_96x128") \
+    X(MYNAH_K_Q5K_GEMM_INT8_128_128, "mynah_q5k_gemm_int8_128x128")
 
 enum {
 #define X(id, name) id,
