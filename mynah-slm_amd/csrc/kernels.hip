@@ -2,8 +2,8 @@
 // translation unit is included here and compiled by a single hipcc --genco).
 //
 // SPDX-License-Identifier: MIT
-#include "dequant.hip"
 #include "gemv_exact.hip"
+#include "dequant.hip"
 #include "gemv_pc.hip"
 #include "gemv_stream.hip"
 #include "gemv_q40.hip"

@@ -192,8 +192,6 @@ int mynah_geometry(int type, size_t rows, size_t cols, size_t *row_bytes) {
 
 /* ── GEMV launch ─────────────────────────────────────────────────────────── */
 
-#define GEMV_WG 256
-
 static int gemv_order = MYNAH_GEMV_EXACT;
 
 int mynah_hip_set_gemv_order(int order) {
@@ -778,15 +776,15 @@ int mynah_dequant_launch(mynah_device *d, int type, const void *w, size_t rows, 
         mynah_set_error("cols must be a multiple of 256");
         return -1;
     }
-    const size_t units = rows * (cols / 32);
-    if (units / GEMV_WG + 1 > 0x7fffffffu) {
+    uint64_t quads = (uint64_t)rows * (cols / 4);
+    const uint64_t grid = (quads + 256u * 4u - 1u) / (256u * 4u);   /* DQ_STEP = 4 */
+    if (grid > 0x7fffffffu) {
         mynah_set_error("dequant too large");
         return -1;
     }
-    uint32_t t = (uint32_t)type, r = (uint32_t)rows, c = (uint32_t)cols;
-    void *args[] = {&w, &y, &t, &r, &c};
-    return mynah_launch(d, MYNAH_K_DEQUANT, (unsigned)((units + GEMV_WG - 1) / GEMV_WG), 1,
-                        GEMV_WG, 0, stream, args);
+    uint32_t t = (uint32_t)type;
+    void *args[] = {&w, &y, &t, &quads};
+    return mynah_launch(d, MYNAH_K_DEQUANT, (unsigned)grid, 1, 256, 0, stream, args);
 }
 
 /* ── host-range registry ─────────────────────────────────────────────────── */
