@@ -932,6 +932,14 @@ static int norm_threads(const mynah_qwen3 *s, const dlayer *L, int ffn, uint32_t
     return rc ? rc : mynah_gemv_group_threads(&g, MYNAH_GEMV_EXACT, thr);
 }
 
+/* Two workgroups of the prefill's scores kernel fit a CU; below twice that a
+ * shorter span fills the chip better than it costs in queries loaded again.
+ * The PV kernel of a quarter of the dimensions reads the probabilities four
+ * times and is the faster one only where whole rows leave CUs idle (63
+ * positions x 16 heads 5.0 against 8.4 us; 2,047 x 32 175 against 153). */
+#define SCORES_WGS 1024u
+#define PV_WGS 512u
+
 /* T tokens (already in pf_tok) at positions s->n_past .. + T - 1 through
  * every layer, filling the cache; no head. */
 static int enqueue_prefill_chunk(mynah_qwen3 *s, mynah_device *d, hipStream_t st, uint32_t T) {
@@ -986,10 +994,17 @@ static int enqueue_prefill_chunk(mynah_qwen3 *s, mynah_device *d, hipStream_t st
             float *sc = s->pf_s, scale = s->scale;
             uint32_t sstride = s->sstride, kvd = s->kv_dim, grp = group;
             uint32_t tt = T;
-            void *args[] = {&qn, &kc, &sc, &p0, &tt, &sstride, &kvd, &grp, &scale};
-            /* 256 positions by 16 queries per workgroup, the queries in LDS */
-            rc = mynah_launch3(d, MYNAH_K_PREFILL_SCORES, c->n_kv_heads, (p0 + T + 255) / 256,
-                               (T + 15) / 16, 256, (size_t)16 * group * 512, st, args);
+            /* Four (32 queries, head) pairs per workgroup, and the most
+             * positions, 128 at most, that still make SCORES_WGS workgroups
+             * (the queries are loaded once per workgroup). */
+            const uint32_t zs = (group * ((T + 31) / 32) + 3) / 4;
+            uint32_t span = (uint32_t)env_or("MYNAH_PREFILL_SPAN", 128) & ~31u;
+            if (span < 32) span = 32;
+            while (span > 32 && c->n_kv_heads * zs * ((p0 + T + span - 1) / span) < SCORES_WGS)
+                span = (span / 2 + 31) & ~31u;
+            void *args[] = {&qn, &kc, &sc, &p0, &tt, &sstride, &kvd, &grp, &scale, &span};
+            rc = mynah_launch3(d, MYNAH_K_PREFILL_SCORES, c->n_kv_heads, (p0 + T + span - 1) / span,
+                               zs, 256, 0, st, args);
             if (rc) break;
             uint32_t nh = c->n_heads;
             void *args2[] = {&sc, &p0, &sstride, &nh};
@@ -998,7 +1013,12 @@ static int enqueue_prefill_chunk(mynah_qwen3 *s, mynah_device *d, hipStream_t st
             const float *vc = vl, *pr = s->pf_s;
             float *out = s->pf_att;
             void *args3[] = {&vc, &pr, &out, &p0, &tt, &sstride, &kvd, &grp};
-            rc = mynah_launch(d, MYNAH_K_PREFILL_PV, c->n_kv_heads, (T + 7) / 8, 512, 0, st, args3);
+            /* Four (16 queries, head) pairs per workgroup; a quarter of the
+             * dimensions where whole rows make too few workgroups. */
+            const uint32_t zp = (group * ((T + 15) / 16) + 3) / 4;
+            const long dims = env_or("MYNAH_PREFILL_PV_DIMS", c->n_kv_heads * zp < PV_WGS ? 32 : 128);
+            rc = mynah_launch3(d, dims == 32 ? MYNAH_K_PREFILL_PV32 : MYNAH_K_PREFILL_PV128,
+                               c->n_kv_heads, zp, dims == 32 ? 4 : 1, 256, 0, st, args3);
         }
         if (rc) break;
         /* src/arch_qwen3.c:223-224: x += Wo attn */

@@ -1570,74 +1570,148 @@ mynah_prefill_rope(float *__restrict__ q, float *__restrict__ k_layer,
     }
 }
 
-// Scores of PS_Q consecutive query rows q0 .. q0 + PS_Q - 1 (positions
-// p0 + q0 + i) against a chunk of PS_POS positions, each lane one position:
-// lane l of wave w holds the whole key row of position t = t0 + 64 w + l in
-// registers and computes, for every (query, head) pair of the tile, the
-// reference's AVX2 dot (src/kernels.c:39-62) in its own registers: the 16
-// FMA chains a[i] = fma(q[16 j + i], k_t[16 j + i], a[i]) over j = 0..7 (a[i]
-// is s0[i] for i < 8, s1[i - 8] otherwise), then tt[i] = a[i] + a[i + 8],
-// v[i] = tt[i] + tt[i + 4], dot = (v0 + v1) + (v2 + v3) -- the operations of
-// the decode kernel's 16-lane form (row16_dot), bit for bit. The query
-// values are wave-uniform LDS reads; the scores of a wave are 64 consecutive
-// floats. A query scores only positions up to its own. Grid (n_kv_heads,
-// ceil((p0 + T) / PS_POS), ceil(T / PS_Q)), block 256; group <= 8.
-#define PS_Q 16
-#define PS_POS 256
-extern "C" __global__ void __launch_bounds__(256)
+// Scores of the chunk's queries against the cache, on the matrix cores. The
+// reference's AVX2 dot (src/kernels.c:39-62) of a query and a key is 16 FMA
+// chains a[i] = fma(q[16 j + i], k_t[16 j + i], a[i]) over j = 0..7 (a[i] is
+// s0[i] for i < 8, s1[i - 8] otherwise), then tt[i] = a[i] + a[i + 8], v[i] =
+// tt[i] + tt[i + 4], dot = (v0 + v1) + (v2 + v3). v_mfma_f32_16x16x4_f32 is
+// exactly such a chain: its four products join the accumulator one after the
+// other in k order, each with fmaf's one rounding (subnormals, infinities and
+// NaN included), so two of them with j as k give chain i of 16 keys x 16
+// queries. Lane l holds of its key (and query) l % 16
+// the values 16 j + i, all i, for j = l / 16 and l / 16 + 4: two runs of 64
+// bytes. Keys are the rows, so lane l receives query l % 16, positions
+// 4 (l / 16) + e, and stores them together; positions past the query's own
+// hold no probability (the softmax masks them).
+// Wave w of workgroup z takes pair block 4 z + w: head pb % group of PS_Q = 32
+// queries from PS_Q (pb / group) on, so the waves of a workgroup read the same
+// keys, span positions (a multiple of PS_CH). PS_CH = 32 keys at a time are
+// copied straight into LDS, whole rows a half wave, one chunk ahead; 16-byte
+// column c of key r sits at c ^ (r % 16), so that the 16 rows of a read are in
+// different banks. Grid (n_kv_heads, ceil((p0 + T) / span), ceil(group ceil(T /
+// PS_Q) / 4)), block 256; the host takes the longest span that still fills the
+// chip.
+// What bounds it: the MFMAs, 32 of 13.6 ns per 256 scores on a SIMD, and 15
+// adds per score beside them. 32 heads over 2,047 positions: 429 -> 207 us
+// (the FMAs on the VALU, queries broadcast from LDS, before; 264 us with the
+// keys read from memory in the operand layout, 16-byte pieces of 64 lines per
+// load).
+#define PS_Q 32
+#define PS_CH 32
+typedef __attribute__((address_space(3))) void pf_lds_void;
+extern "C" __global__ void __launch_bounds__(256, 2)
 mynah_prefill_scores(const float *__restrict__ qn, const float *__restrict__ k_layer,
                      float *__restrict__ scores, uint32_t p0, uint32_t T, uint32_t sstride,
-                     uint32_t kv_dim, uint32_t group, float scale) {
+                     uint32_t kv_dim, uint32_t group, float scale, uint32_t span) {
 #pragma clang fp contract(off)
-    // Queries of the tile, [query][head][128]: PS_Q * group * 512 bytes of
-    // dynamic LDS.
-    extern __shared__ __attribute__((aligned(16))) float ql[];
-    const uint32_t kvh = blockIdx.x, t0 = blockIdx.y * PS_POS, q0 = blockIdx.z * PS_Q;
-    const uint32_t nq = T - q0 < PS_Q ? T - q0 : PS_Q;
-    const uint32_t last = p0 + q0 + nq - 1u;          // position of the tile's last query
-    if (t0 > last) return;
-    const uint32_t n_heads = gridDim.x * group, q_dim = n_heads * 128u;
-    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-    const uint32_t tw = t0 + 64u * wave, t = tw + lane;
-    // Rows past the tile's last query read row 0 (finite, never stored).
-    const float4 *krow = (const float4 *)(k_layer + (size_t)(t <= last ? t : 0u) * kv_dim +
-                                          (size_t)kvh * 128u);
-    float4 k4[32];
-    static_for<32>([&](auto I) { k4[decltype(I)::value] = krow[decltype(I)::value]; });
-    for (uint32_t i = threadIdx.x; i < nq * group * 32u; i += blockDim.x) {
-        const uint32_t qi = i / (group * 32u), rem = i % (group * 32u);
-        *(float4 *)&ql[(qi * group + (rem >> 5)) * 128u + 4u * (rem & 31u)] =
-            *(const float4 *)&qn[(size_t)(q0 + qi) * q_dim + (size_t)kvh * group * 128u + 4u * rem];
+    __shared__ __attribute__((aligned(16))) float kl[2][PS_CH][128];
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t lane = threadIdx.x & 63u, lm = lane & 15u, lk = lane >> 4;
+    const uint32_t kvh = blockIdx.x, n_heads = gridDim.x * group;
+    const uint32_t n_pairs = group * ((T + PS_Q - 1u) / PS_Q), pb = 4u * blockIdx.z + wave;
+    const bool live = pb < n_pairs;
+    const uint32_t q0 = PS_Q * ((live ? pb : n_pairs - 1u) / group), h = kvh * group + pb % group;
+    // The last position that any wave of the workgroup needs, and this wave's.
+    const uint32_t pb_end = 4u * blockIdx.z + 3u < n_pairs ? 4u * blockIdx.z + 3u : n_pairs - 1u;
+    const uint32_t qe = PS_Q * (pb_end / group) + PS_Q;
+    const uint32_t n_wg = p0 + (qe < T ? qe : T), t0 = blockIdx.y * span;
+    const uint32_t n_end = p0 + (q0 + PS_Q < T ? q0 + PS_Q : T);
+    if (t0 >= n_wg) return;
+    const uint32_t n_pos = n_wg - t0 < span ? n_wg - t0 : span;
+    // Wave w copies keys 8 w .. + 7 of a chunk, two per instruction; keys past
+    // the workgroup's last position read that one again.
+    auto copy = [&](uint32_t c) __attribute__((always_inline)) {
+        const uint32_t tc = t0 + PS_CH * c, rmax = n_wg - 1u - tc;
+        const __amdgpu_buffer_rsrc_t kr = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(k_layer + (size_t)tc * kv_dim + (size_t)kvh * 128u), 0, 0xffffffffu,
+            0x00020000);
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) {
+            const uint32_t r = 8u * wave + 2u * i + (lane >> 5);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                kr, (pf_lds_void *)&kl[c & 1u][8u * wave + 2u * i][0], 16,
+                4u * (r < rmax ? r : rmax) * kv_dim + 16u * ((lane & 31u) ^ (r & 15u)), 0, 0, 0);
+        }
+    };
+    copy(0);
+    // Of its key and query the lane holds the runs from 16 (l / 16) and from
+    // 64 + 16 (l / 16) on, four float4 each.
+    v4f q[2][8];
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+        const uint32_t qi = q0 + 16u * b + lm;
+        const float *row = qn + ((size_t)(qi < T ? qi : T - 1u) * n_heads + h) * 128u + 16u * lk;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            q[b][i] = *(const v4f *)(row + 4 * i);
+            q[b][4 + i] = *(const v4f *)(row + 64 + 4 * i);
+        }
     }
-    __syncthreads();
-    for (uint32_t qi = 0; qi < nq; qi++) {
-        const uint32_t pos = p0 + q0 + qi;
-        if (tw > pos) continue;                         // wave-uniform
-        float *srow = scores + (size_t)(q0 + qi) * n_heads * sstride;
-        for (uint32_t h = 0; h < group; h++) {
-            const float4 *qh = (const float4 *)&ql[(qi * group + h) * 128u];
-            float a[16];
-            static_for<16>([&](auto I) { a[decltype(I)::value] = 0.0f; });
-            static_for<8>([&](auto J) {
-                constexpr uint32_t j = decltype(J)::value;
-                static_for<4>([&](auto M) {
-                    constexpr uint32_t m = decltype(M)::value;
-                    const float4 qv = qh[4u * j + m], kv = k4[4u * j + m];
-                    a[4u * m + 0u] = __builtin_fmaf(qv.x, kv.x, a[4u * m + 0u]);
-                    a[4u * m + 1u] = __builtin_fmaf(qv.y, kv.y, a[4u * m + 1u]);
-                    a[4u * m + 2u] = __builtin_fmaf(qv.z, kv.z, a[4u * m + 2u]);
-                    a[4u * m + 3u] = __builtin_fmaf(qv.w, kv.w, a[4u * m + 3u]);
-                });
-            });
-            float tt[8];
-            static_for<8>([&](auto I) {
-                constexpr uint32_t i = decltype(I)::value;
-                tt[i] = a[i] + a[i + 8u];
-            });
-            const float v0 = tt[0] + tt[4], v1 = tt[1] + tt[5], v2 = tt[2] + tt[6],
-                        v3 = tt[3] + tt[7];
-            const float dot = (v0 + v1) + (v2 + v3);
-            if (t <= pos) srow[(size_t)(kvh * group + h) * sstride + t] = dot * scale;
+    const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    const uint32_t nc = (n_pos + PS_CH - 1u) / PS_CH;
+    for (uint32_t c = 0; c < nc; c++) {
+        const uint32_t tc = t0 + PS_CH * c;
+        // Chunk c is in for every wave, and every wave is done with the other
+        // buffer.
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        const bool more = c + 1u < nc;
+        if (!live || tc >= n_end) {             // wave-uniform
+            if (more) copy(c + 1u);
+            continue;
+        }
+#pragma unroll
+        for (uint32_t tile = 0; tile < 2; tile++) {
+            v4f k[8];
+            const float *row = &kl[c & 1u][16u * tile + lm][0];
+#pragma unroll
+            for (uint32_t i = 0; i < 4; i++) {
+                k[i] = *(const v4f *)(row + 4u * ((4u * lk + i) ^ lm));
+                k[4 + i] = *(const v4f *)(row + 4u * ((16u + 4u * lk + i) ^ lm));
+            }
+            if (tile == 0) {
+                // Issued behind the first tile's reads: the compiler makes any
+                // LDS read behind a copy wait for it.
+                __builtin_amdgcn_sched_barrier(0);
+                if (more) copy(c + 1u);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            v4f dot[2], hold[2];
+#pragma unroll
+            for (int ic = 0; ic < 4; ic++) {
+                // Chains ic, ic + 4, ic + 8, ic + 12 of both query tiles.
+                v4f a[2][4];
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+#pragma unroll
+                    for (int b = 0; b < 2; b++)
+                        a[b][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[j][ic], q[b][j][ic], zero,
+                                                                       0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+#pragma unroll
+                    for (int b = 0; b < 2; b++)
+                        a[b][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                            k[4 + j][ic], q[b][4 + j][ic], a[b][j], 0, 0, 0);
+#pragma unroll
+                for (int b = 0; b < 2; b++) {
+                    const v4f v = (a[b][0] + a[b][2]) + (a[b][1] + a[b][3]);
+                    // (v0 + v1) + (v2 + v3)
+                    if (ic == 0) dot[b] = v;
+                    else if (ic == 1) dot[b] = dot[b] + v;
+                    else if (ic == 2) hold[b] = v;
+                    else dot[b] = dot[b] + (hold[b] + v);
+                }
+            }
+            // Positions past n_end, within the row (sstride is a multiple of
+            // PS_CH), hold no score that is read.
+#pragma unroll
+            for (int b = 0; b < 2; b++) {
+                const uint32_t qi = q0 + 16u * b + lm;
+                if (qi < T)
+                    *(v4f *)(scores + ((size_t)qi * n_heads + h) * sstride + tc + 16u * tile +
+                             4u * lk) = dot[b] * scale;
+            }
         }
     }
 }
@@ -1653,133 +1727,183 @@ mynah_prefill_softmax(float *scores, uint32_t p0, uint32_t sstride, uint32_t n_h
     softmax_any(row, p0 + blockIdx.x + 1u, row);
 }
 
-// Weighted V sums of PV_Q consecutive query rows for one key head
-// (src/kernels.c:244-249): out[t][h][d] = fma(v_j[d], p_t,h[j], o) for
-// j = 0 .. p0 + t in order, each chain one thread's register. Thread
-// (d = tid % 128, c = tid / 128) owns the chains (query, head) = pairs
-// c, c + 4, ... of the tile. Per chunk of PV_CH positions the probabilities
-// (0 past each query's own last position, which leaves its chain unchanged:
-// fma(v, 0, o) = o for finite v and o != -0, and o never becomes -0 from
-// +0) and the V rows (rows past the tile's last position hold row 0, finite)
-// are staged in LDS; the next chunk's V rows and probabilities are fetched
-// into registers while this one is summed. Grid (n_kv_heads,
-// ceil(T / PV_Q)), block 512.
-#define PV_Q 8
-#define PV_CH 64
-// G = group (2 .. 8, the decoder's limits): each thread owns NPT = 2 G
-// (query, head) pairs, all compile-time indices; pairs of a short last tile
-// have probabilities 0 (their outputs are not stored).
-template <uint32_t G>
-MYNAH_DEV void prefill_pv_tile(const float *__restrict__ v_layer, const float *__restrict__ probs,
-                               float *__restrict__ out, uint32_t p0, uint32_t T, uint32_t sstride,
-                               uint32_t kv_dim, float (*pl)[PV_CH], float (*vl)[128]) {
+// Weighted V sums of the chunk's queries (src/kernels.c:244-249): out[t][h][d]
+// = fma(v_j[d], p_t,h[j], o) for j = 0 .. p0 + t in order, on the matrix cores:
+// v_mfma_f32_16x16x4_f32 extends the chains of 16 dimensions x 16 queries by
+// four positions in order (the chain property, see mynah_prefill_scores). A
+// wave owns 16 queries of one head (pair block pb as there, PV_Q = 16) and the
+// ND dimensions from d0 = ND blockIdx.z on, in F runs of 16 W: tile m of run f
+// is the dimensions d0 + 16 W f + W r + m, r = 0..15, so one read of W floats
+// of V feeds W tiles, and lane l ends with query l % 16, dimensions d0 + 16 W f
+// + W (4 (l / 16) + e) + m: W consecutive ones per e.
+// V is copied chunk by chunk (PV_CH positions) straight into LDS, one chunk
+// ahead, shared by the workgroup's waves; each wave stages its own
+// probabilities, fetched a chunk ahead in registers. The positions that not
+// every query of the wave may see (its own 16 and up to three before them) are
+// added on the VALU, each lane only up to its query's own position, so no
+// value of a later token touches an earlier one's sum.
+// Workgroups with the most positions start first. Grid (n_kv_heads,
+// ceil(group ceil(T / PV_Q) / 4), 128 / ND), block 256.
+// What bounds it: the MFMAs, 8 of 13.6 ns per 4 positions and 16 queries on a
+// SIMD. 32 heads over 2,047 positions: 493 -> 153 us (one VALU chain per
+// lane, probabilities broadcast from LDS, before).
+#define PV_Q 16
+#define PV_CH 32
+#define PV_LD (PV_CH + 4)
+template <uint32_t ND>
+MYNAH_DEV void prefill_pv(const float *__restrict__ v_layer, const float *__restrict__ probs,
+                          float *__restrict__ out, uint32_t p0, uint32_t T, uint32_t sstride,
+                          uint32_t kv_dim, uint32_t group) {
 #pragma clang fp contract(off)
-    constexpr uint32_t NPT = PV_Q * G / 4u, NPR = PV_Q * G * PV_CH / 512u;
-    const uint32_t kvh = blockIdx.x, q0 = blockIdx.y * PV_Q;
-    const uint32_t nq = T - q0 < PV_Q ? T - q0 : PV_Q;
-    const uint32_t npair = nq * G, n_heads = gridDim.x * G;
-    const uint32_t tid = threadIdx.x, d = tid & 127u, c = tid >> 7;
-    const uint32_t n_end = p0 + q0 + nq;            // positions of the last query
-    const float *vbase = v_layer + (size_t)kvh * 128u;
-    // V fetch role: float4 f = tid + 512 k of the chunk: row f / 32, column
-    // 4 (f % 32); rows past n_end read row 0 (never used). Probability fetch
-    // role: entry i = tid + 512 k of the chunk's PV_Q G x PV_CH (pair i /
-    // PV_CH, position i % PV_CH), 0 past the pair's query or past npair.
-    // Four named registers rather than an array: an array of float4 written
-    // through the compile-time loop stays in private memory.
-    float4 vr0, vr1, vr2, vr3;
-    auto vr = [&](auto K) -> float4 & {
-        constexpr uint32_t k = decltype(K)::value;
-        if constexpr (k == 0) return vr0;
-        else if constexpr (k == 1) return vr1;
-        else if constexpr (k == 2) return vr2;
-        else return vr3;
+    constexpr uint32_t W = ND < 64u ? ND / 16u : 4u, F = ND / (16u * W), RP = 256u / ND;
+    typedef float vw __attribute__((ext_vector_type(W)));
+    __shared__ __attribute__((aligned(16))) float vl[2][PV_CH][ND];
+    __shared__ __attribute__((aligned(16))) float pl[4][PV_Q][PV_LD];
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t lane = threadIdx.x & 63u, lm = lane & 15u, lk = lane >> 4;
+    const uint32_t kvh = blockIdx.x, n_heads = gridDim.x * group;
+    const uint32_t blk = gridDim.y - 1u - blockIdx.y, pb = 4u * blk + wave;
+    const uint32_t n_pairs = group * ((T + PV_Q - 1u) / PV_Q);
+    const bool live = pb < n_pairs;
+    const uint32_t q0 = PV_Q * ((live ? pb : n_pairs - 1u) / group);
+    const uint32_t h = kvh * group + pb % group;
+    // The last position any wave of the workgroup needs, and this wave's.
+    const uint32_t pb_end = 4u * blk + 3u < n_pairs ? 4u * blk + 3u : n_pairs - 1u;
+    const uint32_t qe = PV_Q * (pb_end / group) + PV_Q;
+    const uint32_t n_wg = p0 + (qe < T ? qe : T);
+    const uint32_t n_end = p0 + (q0 + PV_Q < T ? q0 + PV_Q : T);
+    const uint32_t n_all = (p0 + q0 + 1u) & ~3u;     // seen by every query of the wave
+    const uint32_t qi = q0 + lm, n_own = p0 + qi + 1u;
+    // V copy: 1 KiB (RP rows) per instruction, wave w the rows 8 w .. + 7 of the
+    // chunk; rows past the workgroup's last position read that one again.
+    const float *vcol = v_layer + (size_t)kvh * 128u + ND * blockIdx.z;
+    auto copy = [&](uint32_t c) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(vcol + (size_t)(PV_CH * c) * kv_dim), 0, 0xffffffffu, 0x00020000);
+        const uint32_t rmax = n_wg - 1u - PV_CH * c;
+#pragma unroll
+        for (uint32_t i = 0; i < 8u / RP; i++) {
+            const uint32_t r0 = 8u * wave + RP * i, r = r0 + lane / (ND / 4u);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                vr, (pf_lds_void *)&vl[c & 1u][r0][0], 16,
+                4u * (r < rmax ? r : rmax) * kv_dim + 16u * (lane % (ND / 4u)), 0, 0, 0);
+        }
     };
-    float pr_r[NPR];
-    float o[NPT];
-    static_for<NPT>([&](auto K) { o[decltype(K)::value] = 0.0f; });
-    for (uint32_t t0 = 0; t0 < n_end; t0 += PV_CH) {
-        if (t0 == 0) {
-            static_for<4>([&](auto K) {
-                constexpr uint32_t k = decltype(K)::value;
-                const uint32_t f = tid + 512u * k, r = f >> 5;
-                vr(K) = *(const float4 *)(vbase + (size_t)(r < n_end ? r : 0u) * kv_dim + 4u * (f & 31u));
-            });
-            static_for<NPR>([&](auto K) {
-                constexpr uint32_t k = decltype(K)::value;
-                const uint32_t i = tid + 512u * k, pr = i / PV_CH, t = i % PV_CH;
-                const uint32_t qi = pr / G, h = pr % G;
-                pr_r[k] = pr < npair && t < p0 + q0 + qi + 1u
-                              ? probs[((size_t)(q0 + qi) * n_heads + kvh * G + h) * sstride + t]
-                              : 0.0f;
-            });
+    // Probabilities: lane l of query row l / 4 the positions 8 (l % 4) .. + 7
+    // of the chunk (within the row: sstride is a multiple of PV_CH).
+    const uint32_t pq = q0 + (lane >> 2);
+    const float *prow = probs + ((size_t)(pq < T ? pq : T - 1u) * n_heads + h) * sstride +
+                        8u * (lane & 3u);
+    v4f pr[2];
+    auto fetch = [&](uint32_t c) __attribute__((always_inline)) {
+        if (live && PV_CH * c < n_end) {
+            pr[0] = *(const v4f *)(prow + PV_CH * c);
+            pr[1] = *(const v4f *)(prow + PV_CH * c + 4);
         }
+    };
+    const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    v4f acc[F][W];
+#pragma unroll
+    for (uint32_t f = 0; f < F; f++)
+#pragma unroll
+        for (uint32_t m = 0; m < W; m++) acc[f][m] = zero;
+    copy(0);
+    fetch(0);
+    const uint32_t nc = (n_wg + PV_CH - 1u) / PV_CH;
+    for (uint32_t c = 0; c < nc; c++) {
+        *(v4f *)&pl[wave][lane >> 2][8u * (lane & 3u)] = pr[0];
+        *(v4f *)&pl[wave][lane >> 2][8u * (lane & 3u) + 4u] = pr[1];
+        // Chunk c of V (copied a chunk ago) is in for every wave, and every
+        // wave is done with the other buffer.
+        __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
-        static_for<4>([&](auto K) {
-            constexpr uint32_t k = decltype(K)::value;
-            const uint32_t f = tid + 512u * k;
-            *(float4 *)&vl[f >> 5][4u * (f & 31u)] = vr(K);
-        });
-        static_for<NPR>([&](auto K) {
-            constexpr uint32_t k = decltype(K)::value;
-            const uint32_t i = tid + 512u * k;
-            pl[i / PV_CH][i % PV_CH] = pr_r[k];
-        });
-        __syncthreads();
-        const uint32_t t1 = t0 + PV_CH;
-        if (t1 < n_end) {
-            static_for<4>([&](auto K) {
-                constexpr uint32_t k = decltype(K)::value;
-                const uint32_t f = tid + 512u * k, r = t1 + (f >> 5);
-                vr(K) = *(const float4 *)(vbase + (size_t)(r < n_end ? r : 0u) * kv_dim + 4u * (f & 31u));
-            });
-            static_for<NPR>([&](auto K) {
-                constexpr uint32_t k = decltype(K)::value;
-                const uint32_t i = tid + 512u * k, pr = i / PV_CH, t = t1 + i % PV_CH;
-                const uint32_t qi = pr / G, h = pr % G;
-                pr_r[k] = pr < npair && t < p0 + q0 + qi + 1u
-                              ? probs[((size_t)(q0 + qi) * n_heads + kvh * G + h) * sstride + t]
-                              : 0.0f;
-            });
+        const uint32_t tc = PV_CH * c;
+        const bool more = c + 1u < nc;
+        const float(*vc)[ND] = vl[c & 1u];
+        const float *pc = pl[wave][lm];
+        const uint32_t full = !live || n_all <= tc ? 0u : n_all - tc < PV_CH ? n_all - tc : PV_CH;
+        float p[4];
+        vw v[4][F];
+        auto read = [&](uint32_t i, uint32_t j) __attribute__((always_inline)) {
+            p[i] = pc[j + lk];
+#pragma unroll
+            for (uint32_t f = 0; f < F; f++)
+                v[i][f] = *(const vw *)&vc[j + lk][16u * W * f + W * lm];
+        };
+        auto step = [&](uint32_t i) __attribute__((always_inline)) {
+#pragma unroll
+            for (uint32_t f = 0; f < F; f++)
+#pragma unroll
+                for (uint32_t m = 0; m < W; m++)
+                    acc[f][m] =
+                        __builtin_amdgcn_mfma_f32_16x16x4f32(v[i][f][m], p[i], acc[f][m], 0, 0, 0);
+        };
+        // The next chunk's copies are issued behind the first half's reads: the
+        // compiler makes any LDS read behind a copy wait for it.
+        if (full == PV_CH) {
+#pragma unroll
+            for (uint32_t i = 0; i < 4; i++) read(i, 4u * i);
         }
-        // Four positions per step (rounded up: the padding has p = 0).
-        const uint32_t tn = n_end - t0 < PV_CH ? n_end - t0 : PV_CH;
-        for (uint32_t j = 0; j < tn; j += 4) {
-            const float v0 = vl[j][d], v1 = vl[j + 1][d], v2 = vl[j + 2][d], v3 = vl[j + 3][d];
-            static_for<NPT>([&](auto K) {
-                constexpr uint32_t k = decltype(K)::value;
-                const float4 pp = *(const float4 *)&pl[c + 4u * k][j];
-                float acc = o[k];
-                acc = __builtin_fmaf(v0, pp.x, acc);
-                acc = __builtin_fmaf(v1, pp.y, acc);
-                acc = __builtin_fmaf(v2, pp.z, acc);
-                o[k] = __builtin_fmaf(v3, pp.w, acc);
-            });
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) {
+            copy(c + 1u);
+            fetch(c + 1u);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (full == PV_CH) {
+#pragma unroll
+            for (uint32_t i = 0; i < 4; i++) step(i);
+#pragma unroll
+            for (uint32_t i = 0; i < 4; i++) read(i, 16u + 4u * i);
+#pragma unroll
+            for (uint32_t i = 0; i < 4; i++) step(i);
+            continue;
+        }
+        if (!live || tc >= n_end) continue;              // wave-uniform
+#pragma nounroll
+        for (uint32_t j = 0; j < full; j += 4u) {
+            read(0, j);
+            step(0);
+        }
+        const uint32_t stop = n_end - tc < PV_CH ? n_end - tc : PV_CH;
+        for (uint32_t j = full; j < stop; j += 4u) {
+            const v4f ps = *(const v4f *)&pc[j];
+#pragma unroll
+            for (uint32_t f = 0; f < F; f++)
+#pragma unroll
+                for (uint32_t e = 0; e < 4; e++) {
+                    vw u[4];
+#pragma unroll
+                    for (uint32_t i = 0; i < 4; i++)
+                        u[i] = *(const vw *)&vc[j + i][16u * W * f + W * (4u * lk + e)];
+#pragma unroll
+                    for (uint32_t i = 0; i < 4; i++)
+#pragma unroll
+                        for (uint32_t m = 0; m < W; m++) {
+                            const float o = __builtin_fmaf(u[i][m], ps[i], acc[f][m][e]);
+                            acc[f][m][e] = tc + j + i < n_own ? o : acc[f][m][e];
+                        }
+                }
         }
     }
-    static_for<NPT>([&](auto K) {
-        constexpr uint32_t k = decltype(K)::value;
-        const uint32_t pr = c + 4u * k;
-        if (pr < npair) {
-            const uint32_t qi = pr / G, h = pr % G;
-            out[((size_t)(q0 + qi) * n_heads + kvh * G + h) * 128u + d] = o[k];
+    if (!live || qi >= T) return;
+    float *o = out + ((size_t)qi * n_heads + h) * 128u + ND * blockIdx.z + 4u * W * lk;
+#pragma unroll
+    for (uint32_t f = 0; f < F; f++)
+#pragma unroll
+        for (uint32_t e = 0; e < 4; e++) {
+            vw v;
+#pragma unroll
+            for (uint32_t m = 0; m < W; m++) v[m] = acc[f][m][e];
+            *(vw *)(o + 16u * W * f + W * e) = v;
         }
-    });
 }
-
-extern "C" __global__ void __launch_bounds__(512)
-mynah_prefill_pv(const float *__restrict__ v_layer, const float *__restrict__ probs,
-                 float *__restrict__ out, uint32_t p0, uint32_t T, uint32_t sstride,
-                 uint32_t kv_dim, uint32_t group) {
-    __shared__ __attribute__((aligned(16))) float pl[PV_Q * 8][PV_CH];
-    __shared__ __attribute__((aligned(16))) float vl[PV_CH][128];
-    switch (group) {
-    case 2u: prefill_pv_tile<2>(v_layer, probs, out, p0, T, sstride, kv_dim, pl, vl); break;
-    case 3u: prefill_pv_tile<3>(v_layer, probs, out, p0, T, sstride, kv_dim, pl, vl); break;
-    case 4u: prefill_pv_tile<4>(v_layer, probs, out, p0, T, sstride, kv_dim, pl, vl); break;
-    case 5u: prefill_pv_tile<5>(v_layer, probs, out, p0, T, sstride, kv_dim, pl, vl); break;
-    case 6u: prefill_pv_tile<6>(v_layer, probs, out, p0, T, sstride, kv_dim, pl, vl); break;
-    case 7u: prefill_pv_tile<7>(v_layer, probs, out, p0, T, sstride, kv_dim, pl, vl); break;
-    default: prefill_pv_tile<8>(v_layer, probs, out, p0, T, sstride, kv_dim, pl, vl); break;
+#define PV_KERNEL(ND, OCC)                                                                    \
+    extern "C" __global__ void __launch_bounds__(256, OCC) mynah_prefill_pv##ND(              \
+        const float *__restrict__ v_layer, const float *__restrict__ probs,                   \
+        float *__restrict__ out, uint32_t p0, uint32_t T, uint32_t sstride, uint32_t kv_dim,  \
+        uint32_t group) {                                                                     \
+        prefill_pv<ND>(v_layer, probs, out, p0, T, sstride, kv_dim, group);                   \
     }
-}
+PV_KERNEL(128, 3)      // 63 positions x 16 heads: 8.4 us, 2,047 x 32: 153 us
+PV_KERNEL(32, 4)       // 63 positions x 16 heads: 5.0 us, 2,047 x 32: 175 us

@@ -86,7 +86,8 @@ enum { MYNAH_Q4_0 = 2, MYNAH_Q8_0 = 8, MYNAH_Q4_K = 12, MYNAH_Q5_K = 13, MYNAH_Q
     X(MYNAH_K_PREFILL_ROPE, "mynah_prefill_rope")      \
     X(MYNAH_K_PREFILL_SCORES, "mynah_prefill_scores")  \
     X(MYNAH_K_PREFILL_SOFTMAX, "mynah_prefill_softmax") \
-    X(MYNAH_K_PREFILL_PV, "mynah_prefill_pv")          \
+    X(MYNAH_K_PREFILL_PV128, "mynah_prefill_pv128")    \
+    X(MYNAH_K_PREFILL_PV32, "mynah_prefill_pv32")      \
     X(MYNAH_K_COPY16, "mynah_copy16")                  \
     X(MYNAH_K_READ16, "mynah_read16")                  \
     X(MYNAH_K_VALU_ADD_RATE, "mynah_valu_add_rate")  \
