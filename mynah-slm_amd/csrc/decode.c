@@ -81,6 +81,7 @@ struct mynah_qwen3 {
     float *k_cache, *v_cache, *rope_cos, *rope_sin;
     float *rope_now;          /* cos | sin of the position the next step writes (2 x hd / 2) */
     float *x, *q, *attn, *act, *logits, *scores;
+    float *k_now;             /* the step's unrotated key (attn_short) */
     uint32_t *counters;             /* token, pos, step, forced-token count */
     uint32_t *forced;               /* prompt tokens replayed before greedy steps */
     unsigned long long *keys;       /* head workgroups' argmax keys */
@@ -204,7 +205,7 @@ void mynah_hip_qwen3_free(mynah_qwen3 *s) {
             if (s->graph[v][b]) (void)hipGraphDestroy(s->graph[v][b]);
         }
     void *bufs[] = {s->keys, s->blob, s->k_cache, s->v_cache, s->rope_cos, s->rope_sin, s->rope_now,
-                    s->x, s->q,
+                    s->x, s->q, s->k_now,
                     s->attn, s->act, s->logits, s->scores, s->counters, s->tokens, s->forced, s->pm, s->pl,
                     s->po, s->pf_x, s->pf_xn, s->pf_q, s->pf_att, s->pf_g, s->pf_u, s->pf_s,
                     s->pf_tok};
@@ -331,6 +332,7 @@ mynah_qwen3 *mynah_qwen3_new_parts(const mynah_qwen3_shape *c, const mynah_synth
     s->rope_now = (float *)dalloc(2 * half * 4, &ok);
     s->x = (float *)dalloc(dm * 4, &ok);
     s->q = (float *)dalloc((size_t)s->q_dim * 4, &ok);
+    s->k_now = (float *)dalloc((size_t)s->kv_dim * 4, &ok);
     s->attn = (float *)dalloc((size_t)s->q_dim * 4, &ok);
     s->act = (float *)dalloc(ff * 4, &ok);
     s->logits = (float *)dalloc((size_t)c->vocab * 4, &ok);
@@ -411,7 +413,8 @@ static int gemv_desc(mynah_gemv_desc *g, const dtensor *w, const float *x, float
 }
 
 /* The grouped GEMV launches of layer l: LG_QKV q/k/v with the attention
- * norm in front and K/V written into the cache slot at the position,
+ * norm in front and K/V written into the cache slot at the position (K to
+ * k_now where the attention is one launch, which writes the slot itself),
  * LG_O the output projection onto the residual, LG_FFN gate/up with the FFN
  * norm in front and SwiGLU behind, LG_DOWN the down projection onto the
  * residual. */
@@ -536,6 +539,13 @@ static int pv_kernel(const mynah_qwen3 *s, uint32_t cap) {
     return by_cols[(cap - 1u) / col];
 }
 
+/* Whether a launch sized for `cap` positions takes the exact attention in one
+ * launch: up to 256 positions it saves 2.4 - 3.7 us a layer; at 300 - 500 a
+ * form for 512 positions ran level to 0.9 us slower at 0.6B (decode.hip). */
+static int attn_short(const mynah_qwen3 *s, uint32_t cap) {
+    return s->attn_mode != MYNAH_ATTN_SPLIT && cap <= MYNAH_ATTN_SHORT_N && pv_kernel(s, cap) >= 0;
+}
+
 static uint32_t prefetch_step(void) {
     const long v = env_or("MYNAH_PREFETCH_STEP", 7);
     return v >= 2 && v <= 12 ? (uint32_t)v : 7u;
@@ -549,6 +559,7 @@ static int enqueue_step(mynah_qwen3 *s, mynah_device *d, hipStream_t st, int var
     const size_t per_layer = (size_t)s->n_ctx * s->kv_dim;
     uint32_t *tok = TOKEN(s), *pos = POS(s), *step = STEP(s);
     uint32_t head_tiles = 0;
+    const int one = attn_short(s, cap);
     const uint32_t pf_wgs = prefetch_wgs(), pf_step = prefetch_step();
     const long pf_bpw = env_or("MYNAH_PREFETCH_BPW", 8192);
     const long pf_max = env_or("MYNAH_PREFETCH_MAX", 6L << 20);
@@ -594,9 +605,28 @@ static int enqueue_step(mynah_qwen3 *s, mynah_device *d, hipStream_t st, int var
             if (nx) rc = mynah_gemv_prefetch_plan(nx, -1, pf_wgs, pf_b, pf_m, pf_step, &lg[k].pf);
         }
         if (rc) break;
+        if (one) {      /* the raw key to k_now, not the cache slot */
+            lg[LG_QKV].d[1].y = s->k_now;
+            lg[LG_QKV].d[1].ypos = NULL;
+            lg[LG_QKV].d[1].ystride = 0;
+        }
         rc = mynah_gemv_group_launch(d, &lg[LG_QKV], st, NULL, -1);
         if (rc) break;
-        if (s->attn_mode == MYNAH_ATTN_SPLIT) {
+        if (one) {
+            const float *q = s->q, *know = s->k_now, *rnow = s->rope_now, *cvl = vl;
+            const float *qn = (const float *)L->q_norm.dev, *kn = (const float *)L->k_norm.dev;
+            float *out = s->attn, eps = c->rms_eps, scale = s->scale;
+            uint32_t nctx = cap, kvd = s->kv_dim, nkv = c->n_kv_heads;
+            uint32_t group = c->n_heads / c->n_kv_heads;
+            /* Positions live at the launch's first step stay live in every
+             * later one (the graphs replay forward): their rows are loaded
+             * before the position arrives. */
+            uint32_t spec = p0 + 1u;
+            void *args[] = {&q, &know, &kl, &cvl, &qn, &kn, &rnow, &pos, &out,
+                            &nctx, &kvd, &nkv, &group, &eps, &scale, &spec};
+            rc = mynah_launch(d, MYNAH_K_ATTN_SHORT, c->n_heads * (128u / MYNAH_PV_SW), 1, 512, 0,
+                              st, args);
+        } else if (s->attn_mode == MYNAH_ATTN_SPLIT) {
             const float *q = s->q, *qn = (const float *)L->q_norm.dev;
             const float *kn = (const float *)L->k_norm.dev;
             const float *rnow = s->rope_now;

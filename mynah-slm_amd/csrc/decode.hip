@@ -886,6 +886,199 @@ DPV_KERNEL(false, 4, mynah_attn_pv_4)
 // Probabilities from memory (any length).
 DPV_KERNEL(true, 1, mynah_attn_pv_m)
 
+// ── exact attention over a short context, in one launch ────────────────────
+// The scores, the softmax and the PV chain of the two launches above with the
+// same operations in the same order, for n_kv <= ASH_N: a workgroup takes one
+// query head and DPV_SW of its dimensions and computes the head's whole score
+// row itself. What a short context costs is not work but the second launch:
+// its gap and ramp, the position and the score rows read back, three barriers.
+// Each of the 8 slices reads the head's K from the L2 (512 B per position and
+// workgroup), which costs less than the launch up to about 256 positions.
+// Decode step per layer, MI355X, both launches -> this one: 0.6B from 8
+// positions 31.1 -> 28.2 us, from 180 32.9 -> 30.5; 4B 54.0 -> 50.4, 55.4 ->
+// 52.6. Compiled for 512 positions (four passes): from 300 33.0 -> 33.0 (0.6B)
+// and 55.8 -> 55.0 (4B), from 440 34.4 -> 35.3 and 57.4 -> 57.4; so it ends at
+// 256.
+//
+// Eight waves; wave w holds positions 128 p + 16 w .. + 15 of pass p, four
+// lanes a position. Lane quarter m keeps k_t[16 j + 4 m .. + 3] (one float4 a
+// j, so a wave's load takes 64 bytes of 16 rows) and the reference's dot
+// chains 4 m .. 4 m + 3; the horizontal sums are two quad permutes and the
+// last three adds in the lane. The same lanes carry the slice's V of the same
+// positions into LDS, dimension-major (rows of ASH_N + 36 floats: the
+// transposing stores hit 64 distinct banks, the chain's 16-byte reads 16
+// distinct groups). Waves whose positions are below `spec` (live when the
+// launch was enqueued) load before the position arrives. Wave 0 normalises
+// and rotates the query head, wave 1 the new key; its raw projection comes in
+// k_now and not in the cache slot, because every workgroup of the key head
+// reads it while the first one writes the rotated key there (the row at the
+// position is never used from the cache here). After the second barrier wave
+// 0 alone takes the softmax (two values a lane and pass) and the chain. Grid
+// and workgroup order as mynah_attn_pv_*; block 512; hd == 128.
+#define ASH_NP 2
+#define ASH_N (128u * ASH_NP)                             // = MYNAH_ATTN_SHORT_N
+extern "C" __global__ void __launch_bounds__(512)
+mynah_attn_short(const float *q, const float *k_now, float *k_layer, const float *v_layer,
+                 const float *__restrict__ q_norm, const float *__restrict__ k_norm,
+                 const float *__restrict__ rope_now, const uint32_t *__restrict__ pos_ptr,
+                 float *__restrict__ out, uint32_t n_ctx, uint32_t kv_dim, uint32_t n_kv_heads,
+                 uint32_t group, float eps, float scale, uint32_t spec) {
+#pragma clang fp contract(off)
+    constexpr uint32_t VST = ASH_N + 36u;
+    __shared__ __attribute__((aligned(16))) float qn[128], kn[128];
+    __shared__ __attribute__((aligned(16))) float vt[DPV_SW * VST];       // [dim][t]
+    __shared__ __attribute__((aligned(16))) float pl[ASH_N + 32u];        // read ahead past ASH_N
+    __shared__ uint64_t etab[32];
+    const uint32_t forced = index_sums_forced();
+    const uint32_t b = blockIdx.x, kvh = b % n_kv_heads, rest = b / n_kv_heads;
+    const uint32_t head = kvh * group + rest % group, slice = rest / group;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    const uint32_t m = lane & 3u, tw = 16u * wave, tl = tw + (lane >> 2);
+    const float *kcol = k_layer + (size_t)kvh * 128u + 4u * m;
+    const float *vcol = v_layer + (size_t)kvh * 128u + slice * DPV_SW + 4u * m;
+    v4f kr[ASH_NP][8], vr[ASH_NP];
+    auto fetch = [&](v4f *k8, v4f &v, uint32_t p) __attribute__((always_inline)) {
+        const uint32_t t = 128u * p + tl;
+        const size_t row = (size_t)(t < n_ctx ? t : n_ctx - 1u) * kv_dim;
+#pragma unroll
+        for (uint32_t j = 0; j < 8u; j++) k8[j] = *(const v4f *)(kcol + row + 16u * j);
+        v = *(const v4f *)(vcol + row);
+    };
+    // What the norms read goes out first: wave 0 the query, wave 1 the key.
+    float x0 = 0.0f, x1 = 0.0f, w0 = 0.0f, w1 = 0.0f, cs = 0.0f, sn = 0.0f;
+    if (wave < 2u) {
+        const float *src = wave == 0 ? q + (size_t)head * 128u : k_now + (size_t)kvh * 128u;
+        const float *w = wave == 0 ? q_norm : k_norm;
+        x0 = src[lane];
+        x1 = src[lane + 64u];
+        w0 = w[lane];
+        w1 = w[lane + 64u];
+        cs = rope_now[lane];
+        sn = rope_now[64u + lane];
+    }
+    const uint64_t tv = mynah_exp2_tab[lane & 31u];
+#pragma unroll
+    for (uint32_t p = 0; p < (uint32_t)ASH_NP; p++)
+        if (128u * p + tw < spec) fetch(kr[p], vr[p], p);
+    const uint32_t pos = pos_ptr[0], n_kv = pos + 1u;
+#pragma unroll
+    for (uint32_t p = 0; p < (uint32_t)ASH_NP; p++)
+        if (128u * p + tw >= spec && 128u * p + tw < n_kv) fetch(kr[p], vr[p], p);
+    if (wave < 2u) {
+        float y0, y1;
+        const double r = norm_rope_reg(x0, x1, w0, w1, cs, sn, eps, false, y0, y1);
+        if (MYNAH_UNSETTLED(r, 128u, 1u, forced))
+            (void)norm_rope_reg(x0, x1, w0, w1, cs, sn, eps, true, y0, y1);
+        float *dst = wave == 0 ? qn : kn;
+        dst[lane] = y0;
+        dst[lane + 64u] = y1;
+        if (wave == 0) {
+            etab[lane & 31u] = tv;                    // lanes l and l + 32 write the same value
+        } else if (rest == 0) {
+            float *kpos = k_layer + (size_t)pos * kv_dim + (size_t)kvh * 128u;
+            kpos[lane] = y0;
+            kpos[lane + 64u] = y1;
+        }
+    }
+    __syncthreads();
+    v4f q8[8];
+#pragma unroll
+    for (uint32_t j = 0; j < 8u; j++) q8[j] = *(const v4f *)(qn + 16u * j + 4u * m);
+#pragma unroll
+    for (uint32_t p = 0; p < (uint32_t)ASH_NP; p++) {
+        if (128u * p + tw >= n_kv) continue;
+        const uint32_t t = 128u * p + tl;
+        v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (uint32_t j = 0; j < 8u; j++) {
+            v4f k = kr[p][j];
+            if (t == pos) k = *(const v4f *)(kn + 16u * j + 4u * m);
+#pragma unroll
+            for (int c = 0; c < 4; c++) acc[c] = __builtin_fmaf(q8[j][c], k[c], acc[c]);
+        }
+        // tt[l] = s[l] + s[l + 8], v[l] = tt[l] + tt[l + 4] (row16_dot).
+        float v[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const float tt = acc[c] + dpp_f<0x4E>(acc[c]);
+            v[c] = tt + dpp_f<0xB1>(tt);
+        }
+        const float dot = (v[0] + v[1]) + (v[2] + v[3]);
+        if (m == 0) pl[t] = dot * scale;
+#pragma unroll
+        for (uint32_t c = 0; c < 4u; c++) vt[(4u * m + c) * VST + t] = vr[p][c];
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    // The softmax (src/kernels.c:207-220): position 64 i + lane in e[i];
+    // those at or past n_kv are -inf, whose exponential is 0.
+    constexpr int NE = 2 * ASH_NP;
+    float e[NE], mx = -__builtin_inff();
+#pragma unroll
+    for (int i = 0; i < NE; i++) {
+        const uint32_t t = 64u * i + lane;
+        e[i] = t < n_kv ? pl[t] : -__builtin_inff();
+        mx = fmaxf(mx, e[i]);
+    }
+    mx = wave_max_dpp(mx);
+    double sum = 0.0;
+#pragma unroll
+    for (int i = 0; i < NE; i++) {
+        e[i] = mynah_expf_t(e[i] - mx, etab);
+        sum += (double)e[i];
+    }
+    double r = 1.0 / wave_sum_d(sum);
+    if (MYNAH_UNSETTLED(r, n_kv, 2u, forced)) {
+        double seq = 0.0;
+#pragma unroll
+        for (int i = 0; i < NE; i++) {
+            const uint32_t t0 = 64u * i, cnt = n_kv <= t0 ? 0u : n_kv - t0 < 64u ? n_kv - t0 : 64u;
+#pragma nounroll
+            for (uint32_t j = 0; j < cnt; j++)
+                seq += (double)__int_as_float(__builtin_amdgcn_readlane(__float_as_int(e[i]), j));
+        }
+        r = 1.0 / seq;
+    }
+    const float inv = (float)r;
+#pragma unroll
+    for (int i = 0; i < NE; i++) pl[64u * i + lane] = e[i] * inv;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // The chain: four positions a read, eight groups ahead; the reads past
+    // the last position stay in their arrays and are not used.
+    const float *vd = vt + (lane % DPV_SW) * VST;
+    float acc = 0.0f;
+    float4 rv[8], rp[8];
+#pragma unroll
+    for (uint32_t g = 0; g < 8u; g++) {
+        rv[g] = *(const float4 *)(vd + 4u * g);
+        rp[g] = *(const float4 *)(pl + 4u * g);
+    }
+    const uint32_t n4 = n_kv / 4u, left = n_kv % 4u;
+    uint32_t g0 = 0;
+#pragma nounroll
+    for (; g0 + 8u <= n4; g0 += 8u) {
+        static_for<8>([&](auto gi) __attribute__((always_inline)) {
+            constexpr uint32_t g = decltype(gi)::value;
+            acc = ao_fma4(rv[g], rp[g], acc);
+            rv[g] = *(const float4 *)(vd + 4u * (g0 + 8u + g));
+            rp[g] = *(const float4 *)(pl + 4u * (g0 + 8u + g));
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    }
+    static_for<8>([&](auto gi) __attribute__((always_inline)) {
+        constexpr uint32_t g = decltype(gi)::value;
+        if (g0 + g < n4) {
+            acc = ao_fma4(rv[g], rp[g], acc);
+        } else if (g0 + g == n4) {
+            if (left > 0u) acc = __builtin_fmaf(rv[g].x, rp[g].x, acc);
+            if (left > 1u) acc = __builtin_fmaf(rv[g].y, rp[g].y, acc);
+            if (left > 2u) acc = __builtin_fmaf(rv[g].z, rp[g].z, acc);
+        }
+    });
+    if (lane < DPV_SW) out[(size_t)head * 128u + slice * DPV_SW + lane] = acc;
+}
+
 // ── attention with the positions split across workgroups ───────────────────
 // The same operations as mynah_attn_scores + mynah_attn_out, except that the
 // softmax is taken per chunk of CH positions and the chunks are combined

@@ -64,6 +64,7 @@ enum { MYNAH_Q4_0 = 2, MYNAH_Q8_0 = 8, MYNAH_Q4_K = 12, MYNAH_Q5_K = 13, MYNAH_Q
     X(MYNAH_K_ATTN_PV_3, "mynah_attn_pv_3")            \
     X(MYNAH_K_ATTN_PV_4, "mynah_attn_pv_4")            \
     X(MYNAH_K_ATTN_PV_M, "mynah_attn_pv_m")            \
+    X(MYNAH_K_ATTN_SHORT, "mynah_attn_short")          \
     X(MYNAH_K_ATTN_SPLIT, "mynah_attn_split")          \
     X(MYNAH_K_ATTN_SPLIT_G2_32, "mynah_attn_split_g2_32") \
     X(MYNAH_K_ATTN_SPLIT_G2_64, "mynah_attn_split_g2_64") \
@@ -119,6 +120,8 @@ enum {
 /* Dimensions per workgroup of the exact attention's PV kernel (= PV_SW in
  * decode.hip). */
 #define MYNAH_PV_SW 16
+/* Most positions of the one-launch exact attention (= ASH_N in decode.hip). */
+#define MYNAH_ATTN_SHORT_N 256u
 /* Loader waves of the exact attention's PV kernel (= DPV_LW in decode.hip). */
 #ifndef MYNAH_PV_LW
 #define MYNAH_PV_LW 4
