@@ -334,11 +334,99 @@ MYNAH_DEV void gf_stage(gf_f32x16 &s, gf_f32x16 &acc, const float *v, const uint
     }
 }
 
+// Four registers of the four lane quarters transposed: r[i] of quarter j
+// becomes r[j] of quarter i.
+MYNAH_DEV void gf_transpose(float &r0, float &r1, float &r2, float &r3) {
+    uint32_t a = __float_as_uint(r0), b = __float_as_uint(r1), c = __float_as_uint(r2),
+             d = __float_as_uint(r3);
+    const auto ac = __builtin_amdgcn_permlane32_swap(a, c, false, false);
+    const auto bd = __builtin_amdgcn_permlane32_swap(b, d, false, false);
+    const auto ab = __builtin_amdgcn_permlane16_swap(ac[0], bd[0], false, false);
+    const auto cd = __builtin_amdgcn_permlane16_swap(ac[1], bd[1], false, false);
+    r0 = __uint_as_float(ab[0]);
+    r1 = __uint_as_float(ab[1]);
+    r2 = __uint_as_float(cd[0]);
+    r3 = __uint_as_float(cd[1]);
+}
+
+// gf_stage for a tile whose tokens fill only G of its four 16-token groups:
+// the MFMA's four blocks are four consecutive columns of one group instead of
+// one column of four groups, so a stage takes 16 G MFMAs and their adds where
+// gf_stage takes 64 whatever the tokens. 9728 x 2560 Q4_K, 16 tokens: 67 -> 30
+// us; 2560 x 9728 Q6_K, 70 -> 33; 4096 x 2560 Q5_K, 32 tokens: 39.6 -> 28. Its
+// own kernels: beside gf_stage in one kernel it spills. Block b (lane quarter b) of product (m, g) is step 4 m + b of the
+// summation order; its register 4 b + e joins s[4 g + e], b = 0 .. 3 in order.
+// The weights come decoded with a quarter's own eight columns (see load); one
+// 4 x 4 transpose of registers and quarters per 16 of them puts each step's
+// weight in its quarter.
+template <bool MIXED, bool FOLD32, int G>
+MYNAH_DEV void gf_stage_few(gf_f32x16 &s, gf_f32x16 &acc, float *v, const uint8_t *xs,
+                            uint32_t buf, uint32_t lane) {
+#pragma clang fp contract(off)
+    const gf_f32x16 zero = {};
+    const uint32_t t = lane & 15u, q = lane >> 4;
+    // Step 4 m + b: natural, column 4 m + b = value 8 Q + J of a half, Q = m / 2
+    // % 4, J = 4 (m % 2) + b; MIXED, value 2 m + b / 2 of half b % 2, Q = m / 4,
+    // J = 2 (m % 4) + b / 2. a[m]: this quarter's step of product m.
+    float a[16];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        if constexpr (MIXED) {
+            gf_transpose(v[2 * k], v[8 + 2 * k], v[2 * k + 1], v[8 + 2 * k + 1]);
+            a[k] = v[2 * k];
+            a[4 + k] = v[8 + 2 * k];
+            a[8 + k] = v[2 * k + 1];
+            a[12 + k] = v[8 + 2 * k + 1];
+        } else {
+            gf_transpose(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
+#pragma unroll
+            for (int Q = 0; Q < 4; Q++) a[8 * (k / 2) + 2 * Q + k % 2] = v[4 * k + Q];
+        }
+    }
+    // x of product (m, g): the same step of token 16 g + t.
+    auto fetch = [&](int i) __attribute__((always_inline)) {
+        const uint32_t m = (uint32_t)(i / G), g = (uint32_t)(i % G);
+        const uint32_t c = MIXED ? 8u * (q & 1u) + (m >> 1) : m;
+        const uint32_t e = MIXED ? 2u * (m & 1u) + (q >> 1) : q;
+        return *(const float *)(xs + buf + 4096u * g + 256u * t + 16u * (c ^ t) + 4u * e);
+    };
+    auto product = [&](const float b, int i) __attribute__((always_inline)) {
+        return __builtin_amdgcn_mfma_f32_16x16x1f32(a[i / G], b, zero, 0, 0, 0);
+    };
+    constexpr int N = 16 * G, AHEAD = 4;
+    float xb[AHEAD];
+#pragma unroll
+    for (int i = 0; i < AHEAD; i++) xb[i] = fetch(i);
+    gf_f32x16 pc = product(xb[0], 0);
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        gf_f32x16 pn = pc;
+        if (i + AHEAD < N) xb[i % AHEAD] = fetch(i + AHEAD);
+        if (i + 1 < N) pn = product(xb[(i + 1) % AHEAD], i + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        const int g = i % G;
+#pragma unroll
+        for (int b = 0; b < 4; b++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) s[4 * g + e] = s[4 * g + e] + pc[4 * b + e];
+        __builtin_amdgcn_sched_barrier(0);
+        if (FOLD32 && (i / G) % 8 == 7) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                acc[4 * g + e] = acc[4 * g + e] + s[4 * g + e];
+                s[4 * g + e] = 0.0f;
+            }
+        }
+        pc = pn;
+    }
+}
+
 // KW: the waves of a workgroup that share a row group, each taking every
 // KW-th super-block (the z-th split's units u0 + KW round + kz); the running
 // row total passes from one to the next through LDS after every round, in
-// unit order. KW = 1 keeps it in registers.
-template <class Raw, int ORD, int FMT, uint32_t KW>
+// unit order. KW = 1 keeps it in registers. G: the tile's 16-token groups (4,
+// or fewer where the whole launch has no more tokens).
+template <class Raw, int ORD, int FMT, uint32_t KW, int G = 4>
 MYNAH_DEV void gemm_mfma(const uint8_t *__restrict__ w, const float *__restrict__ x, float *y,
                          uint32_t rows, uint32_t cols, uint32_t tokens, uint32_t row_bytes,
                          const float *res, float *__restrict__ part) {
@@ -375,7 +463,7 @@ MYNAH_DEV void gemm_mfma(const uint8_t *__restrict__ w, const float *__restrict_
     gf_f32x16 acc = zero, s = zero;
     Raw raw;
     if (u0 + kz < u1) {
-        gf_stage_x(xl[kz][0], xr, xo, stage, wave);
+        if (wave < (uint32_t)G) gf_stage_x(xl[kz][0], xr, xo, stage, wave);
         raw.load(blk, q);
     }
     for (uint32_t ub = u0; ub < u1; ub += KW) {
@@ -391,7 +479,7 @@ MYNAH_DEV void gemm_mfma(const uint8_t *__restrict__ w, const float *__restrict_
             __syncthreads();
             if (active) {
                 stage += st == 3u ? 4u * KW - 3u : 1u;
-                if (st < 3u || more) gf_stage_x(xl[kz][(st + 1u) & 1u], xr, xo, stage, wave);
+                if (wave < (uint32_t)G && (st < 3u || more)) gf_stage_x(xl[kz][(st + 1u) & 1u], xr, xo, stage, wave);
                 float v[16];
                 if (st == 0) raw.template decode<0>(q, v);
                 else if (st == 1) raw.template decode<1>(q, v);
@@ -401,8 +489,12 @@ MYNAH_DEV void gemm_mfma(const uint8_t *__restrict__ w, const float *__restrict_
                     blk += (size_t)Raw::UB * KW;
                     if (more) raw.load(blk, q);
                 }
-                gf_stage<ORD == 1 && (FMT == 12 || FMT == 13), FOLD32>(
-                    s, acc, v, (const uint8_t *)xl[kz], xa);
+                constexpr bool MIXED = ORD == 1 && (FMT == 12 || FMT == 13);
+                if constexpr (G == 4)
+                    gf_stage<MIXED, FOLD32>(s, acc, v, (const uint8_t *)xl[kz], xa);
+                else
+                    gf_stage_few<MIXED, FOLD32, G>(s, acc, v, (const uint8_t *)xl[kz],
+                                                   xa & (4u * 64u * GF_TOK), lane);
                 xa ^= 4u * 64u * GF_TOK;
             }
         }
@@ -471,6 +563,25 @@ GEMM_MFMA_ENTRIES(mynah_q80_gemm_exact_mfma, GfQ80, 0, 8)
 GEMM_MFMA_ENTRIES(mynah_q4k_gemm_mv_mfma, GfQ4K, 1, 12)
 GEMM_MFMA_ENTRIES(mynah_q5k_gemm_mv_mfma, GfQ5K, 1, 13)
 GEMM_MFMA_ENTRY(mynah_q80_gemm_mv_mfma1, GfQ80, 1, 8, 1)
+
+// At most 16 G tokens: grid (ceil(rows / 64), 1, Z), block 256.
+#define GEMM_FEW_ENTRY(name, RAW, ORD, FMT, G)                                                \
+    extern "C" __global__ void __launch_bounds__(256, 2)                                       \
+        name(const uint8_t *__restrict__ w, const float *__restrict__ x, float *y,             \
+             uint32_t rows, uint32_t cols, uint32_t tokens, uint32_t row_bytes,                \
+             const float *res, float *part) {                                                  \
+        gemm_mfma<RAW, ORD, FMT, 1, G>(w, x, y, rows, cols, tokens, row_bytes, res, part);     \
+    }
+#define GEMM_FEW_ENTRIES(name, RAW, ORD, FMT)                                                 \
+    GEMM_FEW_ENTRY(name##16, RAW, ORD, FMT, 1)                                                 \
+    GEMM_FEW_ENTRY(name##32, RAW, ORD, FMT, 2)
+GEMM_FEW_ENTRIES(mynah_q4k_gemm_exact_few, GfQ4K, 0, 12)
+GEMM_FEW_ENTRIES(mynah_q5k_gemm_exact_few, GfQ5K, 0, 13)
+GEMM_FEW_ENTRIES(mynah_q6k_gemm_exact_few, GfQ6K, 0, 14)
+GEMM_FEW_ENTRIES(mynah_q80_gemm_exact_few, GfQ80, 0, 8)
+GEMM_FEW_ENTRIES(mynah_q4k_gemm_mv_few, GfQ4K, 1, 12)
+GEMM_FEW_ENTRIES(mynah_q5k_gemm_mv_few, GfQ5K, 1, 13)
+GEMM_FEW_ENTRIES(mynah_q80_gemm_mv_few, GfQ80, 1, 8)
 
 // The in-order fold of split-K unit sums: y[t][r] = (res[t][r] +) the row
 // total continued from part[0][t][r] (the first split's running total over

@@ -44,9 +44,10 @@ static const double gemm_step_ns[3][5] = {{0.0, 54.0, 37.8, 37.3, 33.0},
  * round's length set by its longest split (in rounds of kw units) and the
  * waves per SIMD it leaves; a split costs the fold's traffic (each unit sum
  * past the first split written and read, about 4.5 TB/s) and its launch.
- * cap: most splits. */
+ * cap: most splits. unit_steps: MFMAs of a super-block and wave (256, or 64 a
+ * 16-token group in the kernels for few tokens). */
 static gemm_split gemm_plan(uint64_t tiles, uint32_t units, uint64_t outputs, uint32_t cus,
-                            uint32_t max_kw, uint32_t cap) {
+                            uint32_t max_kw, uint32_t cap, double unit_steps) {
     gemm_split best = {1, 1};
     double best_ns = 0.0;
     for (uint32_t kw = 1, i = 0; kw <= max_kw && kw <= units; kw *= 2u, i++) {
@@ -54,7 +55,7 @@ static gemm_split gemm_plan(uint64_t tiles, uint32_t units, uint64_t outputs, ui
         for (uint32_t nz = 1; nz <= cap && nz <= units; nz++) {
             if (nz > 1 && tiles * (nz - 1u) >= slots) break;
             const uint32_t per = (units + nz - 1u) / nz;
-            const double steps = 256.0 * (double)((per + kw - 1u) / kw);
+            const double steps = unit_steps * (double)((per + kw - 1u) / kw);
             uint64_t left = tiles * nz;
             const uint64_t full = left / slots;
             double ns = (double)full * steps * 4.0 * gemm_step_ns[i][4];
@@ -88,18 +89,30 @@ static int gemm_mfma_launch(mynah_device *d, int type, int ord, const void *w, s
          MYNAH_K_Q80_GEMM_MFMA1},
         {MYNAH_K_Q4K_GEMM_MV_MFMA1, MYNAH_K_Q5K_GEMM_MV_MFMA1, MYNAH_K_Q6K_GEMM_MFMA1,
          MYNAH_K_Q80_GEMM_MV_MFMA1}};
+    static const int fid[2][4] = {
+        {MYNAH_K_Q4K_GEMM_FEW16, MYNAH_K_Q5K_GEMM_FEW16, MYNAH_K_Q6K_GEMM_FEW16,
+         MYNAH_K_Q80_GEMM_FEW16},
+        {MYNAH_K_Q4K_GEMM_MV_FEW16, MYNAH_K_Q5K_GEMM_MV_FEW16, MYNAH_K_Q6K_GEMM_FEW16,
+         MYNAH_K_Q80_GEMM_MV_FEW16}};
     const int ti = type == MYNAH_Q4_K ? 0 : type == MYNAH_Q5_K ? 1 : type == MYNAH_Q6_K ? 2 : 3;
     const uint32_t units = (uint32_t)(cols / 256);
     const unsigned gx = (unsigned)((rows + 63) / 64), gy = (unsigned)((tokens + 63) / 64);
+    /* Up to 32 tokens a tile's empty 16-token groups are not computed: four
+     * columns of one group an MFMA, where the full tile has one column of four
+     * groups. 9728 x 2560 Q4_K, full tile -> few: 2 tokens 64 -> 27 us, 16
+     * 67 -> 30, 32 69 -> 45 (MYNAH_GEMM_FEW=0: always the full tile). */
+    const uint32_t few =
+        tokens <= 32 && env_long("MYNAH_GEMM_FEW", 1) ? (uint32_t)(tokens + 15) / 16 : 0u;
     gemm_split p = {1, 1};
     if (!(ord == 1 && type == MYNAH_Q8_0)) {
         const long cap = env_long("MYNAH_GEMM_SPLIT", 64), kw = env_long("MYNAH_GEMM_KW", 0);
-        p = gemm_plan((uint64_t)gx * gy, units, (uint64_t)rows * tokens, (uint32_t)d->cus, 4u,
-                      cap > 1 ? (uint32_t)cap : 1u);
-        if (kw == 1 || kw == 2 || kw == 4) p.kw = (uint32_t)kw;
+        p = gemm_plan((uint64_t)gx * gy, units, (uint64_t)rows * tokens, (uint32_t)d->cus,
+                      few ? 1u : 4u, cap > 1 ? (uint32_t)cap : 1u, few ? 64.0 * few : 256.0);
+        if (!few && (kw == 1 || kw == 2 || kw == 4)) p.kw = (uint32_t)kw;
     }
     const uint32_t nz = p.nz;
-    const int kernel = kid[ord][ti] + (p.kw == 4 ? 2 : p.kw == 2 ? 1 : 0);
+    const int kernel = few ? fid[ord][ti] + (int)few - 1
+                           : kid[ord][ti] + (p.kw == 4 ? 2 : p.kw == 2 ? 1 : 0);
     const unsigned block = 256u * p.kw;
     uint32_t r32 = (uint32_t)rows, c32 = (uint32_t)cols, t32 = (uint32_t)tokens,
              rb32 = (uint32_t)rb;

@@ -45,6 +45,20 @@ enum { MYNAH_Q4_0 = 2, MYNAH_Q8_0 = 8, MYNAH_Q4_K = 12, MYNAH_Q5_K = 13, MYNAH_Q
     X(MYNAH_K_Q5K_GEMM_MV_MFMA2, "mynah_q5k_gemm_mv_mfma2") \
     X(MYNAH_K_Q5K_GEMM_MV_MFMA4, "mynah_q5k_gemm_mv_mfma4") \
     X(MYNAH_K_Q80_GEMM_MV_MFMA1, "mynah_q80_gemm_mv_mfma1") \
+    X(MYNAH_K_Q4K_GEMM_FEW16, "mynah_q4k_gemm_exact_few16") \
+    X(MYNAH_K_Q4K_GEMM_FEW32, "mynah_q4k_gemm_exact_few32") \
+    X(MYNAH_K_Q5K_GEMM_FEW16, "mynah_q5k_gemm_exact_few16") \
+    X(MYNAH_K_Q5K_GEMM_FEW32, "mynah_q5k_gemm_exact_few32") \
+    X(MYNAH_K_Q6K_GEMM_FEW16, "mynah_q6k_gemm_exact_few16") \
+    X(MYNAH_K_Q6K_GEMM_FEW32, "mynah_q6k_gemm_exact_few32") \
+    X(MYNAH_K_Q80_GEMM_FEW16, "mynah_q80_gemm_exact_few16") \
+    X(MYNAH_K_Q80_GEMM_FEW32, "mynah_q80_gemm_exact_few32") \
+    X(MYNAH_K_Q4K_GEMM_MV_FEW16, "mynah_q4k_gemm_mv_few16") \
+    X(MYNAH_K_Q4K_GEMM_MV_FEW32, "mynah_q4k_gemm_mv_few32") \
+    X(MYNAH_K_Q5K_GEMM_MV_FEW16, "mynah_q5k_gemm_mv_few16") \
+    X(MYNAH_K_Q5K_GEMM_MV_FEW32, "mynah_q5k_gemm_mv_few32") \
+    X(MYNAH_K_Q80_GEMM_MV_FEW16, "mynah_q80_gemm_mv_few16") \
+    X(MYNAH_K_Q80_GEMM_MV_FEW32, "mynah_q80_gemm_mv_few32") \
     X(MYNAH_K_GEMM_FOLD, "mynah_gemm_fold")            \
     X(MYNAH_K_GEMV_GROUP, "mynah_gemv_group")          \
     X(MYNAH_K_GEMV_GROUP_Q6K, "mynah_gemv_group_q6k")  \
