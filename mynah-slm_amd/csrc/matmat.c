@@ -26,6 +26,7 @@ static long env_long(const char *name, long dflt) {
  * memory and are folded in order afterwards (mynah_gemm_fold). */
 typedef struct {
     uint32_t kw, nz;
+    double ns;      /* estimated */
 } gemm_split;
 
 /* Nanoseconds per column step and SIMD with w waves on it, measured on MI355X
@@ -48,8 +49,7 @@ static const double gemm_step_ns[3][5] = {{0.0, 54.0, 37.8, 37.3, 33.0},
  * 16-token group in the kernels for few tokens). */
 static gemm_split gemm_plan(uint64_t tiles, uint32_t units, uint64_t outputs, uint32_t cus,
                             uint32_t max_kw, uint32_t cap, double unit_steps) {
-    gemm_split best = {1, 1};
-    double best_ns = 0.0;
+    gemm_split best = {1, 1, 0.0};
     for (uint32_t kw = 1, i = 0; kw <= max_kw && kw <= units; kw *= 2u, i++) {
         const uint64_t slots = (uint64_t)cus * (4u / kw);
         for (uint32_t nz = 1; nz <= cap && nz <= units; nz++) {
@@ -66,8 +66,8 @@ static gemm_split gemm_plan(uint64_t tiles, uint32_t units, uint64_t outputs, ui
             }
             if (nz > 1)
                 ns += 4000.0 + (double)outputs * 8.0 * (double)(units - units / nz + 1u) / 4500.0;
-            if (best_ns == 0.0 || ns < best_ns) {
-                best_ns = ns;
+            if (best.ns == 0.0 || ns < best.ns) {
+                best.ns = ns;
                 best.kw = kw;
                 best.nz = nz;
             }
@@ -76,13 +76,34 @@ static gemm_split gemm_plan(uint64_t tiles, uint32_t units, uint64_t outputs, ui
     return best;
 }
 
+/* Up to 32 tokens a tile's empty 16-token groups are not computed: four columns
+ * of one group an MFMA, where the full tile has one column of four groups.
+ * 9728 x 2560 Q4_K, full tile -> few: 2 tokens 64 -> 27 us, 16 67 -> 30, 32
+ * 69 -> 45 (MYNAH_GEMM_FEW=0: always the full tile). The groups, or 0. */
+static uint32_t gemm_few(size_t tokens) {
+    return tokens <= 32 && env_long("MYNAH_GEMM_FEW", 1) ? (uint32_t)(tokens + 15) / 16 : 0u;
+}
+
+static gemm_split gemm_split_of(const mynah_device *d, int type, int ord, size_t rows, size_t cols,
+                                size_t tokens) {
+    const uint32_t few = gemm_few(tokens);
+    const uint64_t tiles = (uint64_t)((rows + 63) / 64) * ((tokens + 63) / 64);
+    const double steps = few ? 64.0 * few : 256.0;
+    const uint32_t units = (uint32_t)(cols / 256);
+    /* The Q8_0 matvec order has no unit sums to split by. */
+    const int whole = ord == 1 && type == MYNAH_Q8_0;
+    const long cap = whole ? 1 : env_long("MYNAH_GEMM_SPLIT", 64);
+    return gemm_plan(tiles, units, (uint64_t)rows * tokens, (uint32_t)d->cus,
+                     few || whole ? 1u : 4u, cap > 1 ? (uint32_t)cap : 1u, steps);
+}
+
 /* The exact GEMM with its products on MFMA (gemm_mfma.hip): the default;
  * MYNAH_GEMM_MFMA=0 runs the VALU kernels of gemm_exact.hip instead (same
  * bits). MYNAH_GEMM_SPLIT=0 never splits over gridDim.z, N at most N ways;
  * MYNAH_GEMM_KW=1|2|4 forces kw. */
-static int gemm_mfma_launch(mynah_device *d, int type, int ord, const void *w, size_t rows,
-                            size_t cols, size_t rb, const float *x, float *y, size_t tokens,
-                            const float *res, hipStream_t stream) {
+static int gemm_mfma_part(mynah_device *d, int type, int ord, const void *w, size_t rows,
+                          size_t cols, size_t rb, const float *x, float *y, size_t tokens,
+                          const float *res, gemm_split p, float *part, hipStream_t stream) {
     /* Q6_K sums in one order either way. */
     static const int kid[2][4] = {
         {MYNAH_K_Q4K_GEMM_MFMA1, MYNAH_K_Q5K_GEMM_MFMA1, MYNAH_K_Q6K_GEMM_MFMA1,
@@ -97,47 +118,63 @@ static int gemm_mfma_launch(mynah_device *d, int type, int ord, const void *w, s
     const int ti = type == MYNAH_Q4_K ? 0 : type == MYNAH_Q5_K ? 1 : type == MYNAH_Q6_K ? 2 : 3;
     const uint32_t units = (uint32_t)(cols / 256);
     const unsigned gx = (unsigned)((rows + 63) / 64), gy = (unsigned)((tokens + 63) / 64);
-    /* Up to 32 tokens a tile's empty 16-token groups are not computed: four
-     * columns of one group an MFMA, where the full tile has one column of four
-     * groups. 9728 x 2560 Q4_K, full tile -> few: 2 tokens 64 -> 27 us, 16
-     * 67 -> 30, 32 69 -> 45 (MYNAH_GEMM_FEW=0: always the full tile). */
-    const uint32_t few =
-        tokens <= 32 && env_long("MYNAH_GEMM_FEW", 1) ? (uint32_t)(tokens + 15) / 16 : 0u;
-    gemm_split p = {1, 1};
-    if (!(ord == 1 && type == MYNAH_Q8_0)) {
-        const long cap = env_long("MYNAH_GEMM_SPLIT", 64), kw = env_long("MYNAH_GEMM_KW", 0);
-        p = gemm_plan((uint64_t)gx * gy, units, (uint64_t)rows * tokens, (uint32_t)d->cus,
-                      few ? 1u : 4u, cap > 1 ? (uint32_t)cap : 1u, few ? 64.0 * few : 256.0);
-        if (!few && (kw == 1 || kw == 2 || kw == 4)) p.kw = (uint32_t)kw;
-    }
+    const uint32_t few = gemm_few(tokens);
     const uint32_t nz = p.nz;
     const int kernel = few ? fid[ord][ti] + (int)few - 1
                            : kid[ord][ti] + (p.kw == 4 ? 2 : p.kw == 2 ? 1 : 0);
     const unsigned block = 256u * p.kw;
     uint32_t r32 = (uint32_t)rows, c32 = (uint32_t)cols, t32 = (uint32_t)tokens,
              rb32 = (uint32_t)rb;
-    if (nz <= 1) {
-        float *part = NULL;
-        void *args[] = {&w, &x, &y, &r32, &c32, &t32, &rb32, &res, &part};
-        return mynah_launch3(d, kernel, gx, gy, 1, block, 0, stream, args);
+    void *args[] = {&w, &x, &y, &r32, &c32, &t32, &rb32, &res, &part};
+    int rc = mynah_launch3(d, kernel, gx, gy, nz, block, 0, stream, args);
+    if (rc == 0 && nz > 1) {
+        uint32_t u32 = units, first = units / nz;   /* the units of split 0 */
+        void *fargs[] = {&part, &res, &y, &r32, &t32, &first, &u32};
+        rc = mynah_launch(d, MYNAH_K_GEMM_FOLD, (unsigned)((rows * tokens + 255) / 256), 1, 256, 0,
+                          stream, fargs);
     }
-    const size_t n = rows * tokens, bytes = (size_t)units * n * sizeof(float);
+    return rc;
+}
+
+/* A last tile of at most 32 tokens costs a full one: where the estimates say
+ * so (8 us for the launches more), the tokens before it and these run as two
+ * products, one after the other in one workspace, the second in the kernels
+ * for few tokens. Every output is the same sum either way. 9728 x 2560 Q4_K, 65
+ * tokens: 145 -> 97 us; 201: 246 -> 216; 2560 x 9728 Q6_K, 201: 263 -> 232;
+ * 6144 x 2048 Q4_K, 130: 105 -> 90. Not for the Q8_0 matvec order, which cannot
+ * split the second product (4096 x 2048, 270 tokens: 166 -> 169). */
+static int gemm_mfma_launch(mynah_device *d, int type, int ord, const void *w, size_t rows,
+                            size_t cols, size_t rb, const float *x, float *y, size_t tokens,
+                            const float *res, hipStream_t stream) {
+    const long kw = env_long("MYNAH_GEMM_KW", 0);
+    const int whole = ord == 1 && type == MYNAH_Q8_0;
+    size_t head = tokens, last = tokens % 64;
+    gemm_split ph = gemm_split_of(d, type, ord, rows, cols, tokens), pl = {1, 1, 0.0};
+    if (!whole && last > 0 && last < tokens && gemm_few(last)) {
+        const gemm_split a = gemm_split_of(d, type, ord, rows, cols, tokens - last);
+        pl = gemm_split_of(d, type, ord, rows, cols, last);
+        if (a.ns + pl.ns + 8000.0 < ph.ns) {
+            head = tokens - last;
+            ph = a;
+        }
+    }
+    if (!whole && !gemm_few(head) && (kw == 1 || kw == 2 || kw == 4))
+        ph.kw = (uint32_t)kw;
+    size_t n = ph.nz > 1 ? rows * head : 0;
+    if (head < tokens && pl.nz > 1 && rows * last > n) n = rows * last;
+    const size_t bytes = cols / 256 * n * sizeof(float);
     float *part = NULL;
-    hipError_t e = hipMallocAsync((void **)&part, bytes, stream);
+    hipError_t e = bytes ? hipMallocAsync((void **)&part, bytes, stream) : hipSuccess;
     if (e != hipSuccess) {
         mynah_set_error("hipMallocAsync(split-K partials, %zu bytes): %s", bytes,
                         hipGetErrorString(e));
         return -1;
     }
-    void *args[] = {&w, &x, &y, &r32, &c32, &t32, &rb32, &res, &part};
-    int rc = mynah_launch3(d, kernel, gx, gy, nz, block, 0, stream, args);
-    if (rc == 0) {
-        uint32_t u32 = units, first = units / nz;   /* the units of split 0 */
-        void *fargs[] = {&part, &res, &y, &r32, &t32, &first, &u32};
-        rc = mynah_launch(d, MYNAH_K_GEMM_FOLD, (unsigned)((n + 255) / 256), 1, 256, 0, stream,
-                          fargs);
-    }
-    e = hipFreeAsync(part, stream);
+    int rc = gemm_mfma_part(d, type, ord, w, rows, cols, rb, x, y, head, res, ph, part, stream);
+    if (rc == 0 && head < tokens)
+        rc = gemm_mfma_part(d, type, ord, w, rows, cols, rb, x + head * cols, y + head * rows, last,
+                            res ? res + head * rows : NULL, pl, part, stream);
+    e = bytes ? hipFreeAsync(part, stream) : hipSuccess;
     if (rc == 0 && e != hipSuccess) {
         mynah_set_error("hipFreeAsync(split-K partials): %s", hipGetErrorString(e));
         return -1;

@@ -30,3 +30,18 @@ def test_few_tokens(M, monkeypatch, qtype, mv, rows, units, tokens):  # noqa: F8
         for env in ({}, {"MYNAH_GEMM_SPLIT": "0"}, {"MYNAH_GEMM_SPLIT": "3"}):
             got = product(M, monkeypatch, env, mv, qtype, w, rows, cols, x, tokens, res)
             assert same(got, ref), env
+
+
+@pytest.mark.parametrize("rows,cols,tokens", [(4096, 2560, 65), (4095, 2560, 80), (2048, 2048, 270),
+                                              (2560, 9728, 96)])
+@pytest.mark.parametrize("mv", [False, True])
+@pytest.mark.parametrize("qtype", [12, 13, 14, 8])
+def test_few_tokens_past_the_last_tile(M, monkeypatch, qtype, mv, rows, cols, tokens):  # noqa: F811
+    """Sizes where the tokens past the last whole tile run as a product of their own."""
+    w = M.synth_blocks(qtype, rows, rows, cols)
+    x = M.synth_normal(rows, tokens * cols)
+    res = M.synth_normal(tokens, tokens * rows) if mv else None
+    ref = product(M, monkeypatch, {"MYNAH_GEMM_MFMA": "0"}, mv, qtype, w, rows, cols, x, tokens,
+                  res)
+    got = product(M, monkeypatch, {}, mv, qtype, w, rows, cols, x, tokens, res)
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
