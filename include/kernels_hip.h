@@ -142,7 +142,12 @@ void *mynah_hip_device_ptr(const void *host);
 
 /* Device-pointer twins. Weights 16-byte aligned for Q4_K / Q5_K and 2-byte
  * aligned for Q6_K / Q8_0 / Q4_0 (GGUF data and whole-row offsets satisfy
- * both); x 16-byte aligned. Asynchronous on `stream`. */
+ * both); x 16-byte aligned. Asynchronous on `stream`. An exact batched
+ * product that splits its super-blocks allocates their sums in stream order
+ * (rows * tokens * 4 bytes for all but the first split's super-blocks; at most
+ * 256 MiB where rows x tokens has more 64 x 64 tiles than the GPU has CUs) and
+ * runs unsplit, to the same bits, where it cannot. The int8 lane allocates its
+ * quantised activations the same way. */
 int mynah_hip_matvec_dev(int type, const void *w, size_t rows, size_t cols,
                          const float *x, float *y, void *stream);
 int mynah_hip_matmat_dev(int type, const void *w, size_t rows, size_t cols,

@@ -61,8 +61,8 @@
 // Launches too small to give every SIMD four waves share a tile among more of
 // them, in two ways (the host plans both). KW = 2 or 4 waves per row group: the
 // template below. Split K (gridDim.z > 1): workgroup z takes the units
-// [z U / Z, (z + 1) U / Z); z = 0 stores the running row total of its units (from 0, in order) to
-// part[0][token][row], every other z stores each unit's sum to
+// [z U / Z, (z + 1) U / Z); z = 0 stores the running row total of its units
+// (from 0, in order) to part[0][token][row], every other z stores each unit's sum to
 // part[u][token][row]; mynah_gemm_fold then continues the total from slot 0
 // over the later units in order (and adds res), the row total the single
 // launch would give. Not for the Q8_0 matvec order, whose row total takes
@@ -500,10 +500,11 @@ MYNAH_DEV void gemm_mfma(const uint8_t *__restrict__ w, const float *__restrict_
         }
         if (FOLD32) continue;
         if (split && z > 0u) {
-            // Unit u's sums, for the in-order fold.
+            // Unit u's sums, for the in-order fold: slot 1 + its place past
+            // the first split's units.
             if (active)
-                gf_store(part + (size_t)u * tokens * rows, s, nullptr, rows, tokens, row0, tok0,
-                         (xa >> 8) & 63u);
+                gf_store(part + (size_t)(u - units / nz + 1u) * tokens * rows, s, nullptr, rows,
+                         tokens, row0, tok0, (xa >> 8) & 63u);
         } else if (KW == 1) {
             acc = acc + s;
         } else {
@@ -584,27 +585,27 @@ GEMM_FEW_ENTRIES(mynah_q5k_gemm_mv_few, GfQ5K, 1, 13)
 GEMM_FEW_ENTRIES(mynah_q80_gemm_mv_few, GfQ80, 1, 8)
 
 // The in-order fold of split-K unit sums: y[t][r] = (res[t][r] +) the row
-// total continued from part[0][t][r] (the first split's running total over
-// its units 0 .. first - 1) over part[u][t][r], u = first .. units - 1, in
-// order — the row total of the reference's order. One thread per output,
-// consecutive rows consecutive threads; the loads go out four at a time.
+// total continued from part[0][t][r] (the first split's running total) over
+// part[i][t][r], i = 1 .. slots - 1 (the later units' sums) in order — the row
+// total of the reference's order. One thread per output, consecutive rows
+// consecutive threads; the loads go out four at a time.
 extern "C" __global__ void __launch_bounds__(256)
 mynah_gemm_fold(const float *__restrict__ part, const float *res, float *y, uint32_t rows,
-                uint32_t tokens, uint32_t first, uint32_t units) {
+                uint32_t tokens, uint32_t slots) {
 #pragma clang fp contract(off)
     const uint64_t n = (uint64_t)rows * tokens;
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     float acc = part[i];
-    uint32_t u = first;
-    for (; u + 4u <= units; u += 4u) {
+    uint32_t u = 1u;
+    for (; u + 4u <= slots; u += 4u) {
         float v[4];
 #pragma unroll
         for (uint32_t k = 0; k < 4; k++) v[k] = part[(size_t)(u + k) * n + i];
 #pragma unroll
         for (uint32_t k = 0; k < 4; k++) acc = acc + v[k];
     }
-    for (; u < units; u++) acc = acc + part[(size_t)u * n + i];
+    for (; u < slots; u++) acc = acc + part[(size_t)u * n + i];
     y[i] = res ? res[i] + acc : acc;
 }
 

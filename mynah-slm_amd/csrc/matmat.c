@@ -29,6 +29,27 @@ typedef struct {
     double ns;      /* estimated */
 } gemm_split;
 
+/* Partial sums of a split launch, per output: the first split's running total
+ * and one sum per unit of the later splits (0: nothing goes through memory). */
+static uint32_t gemm_slots(uint32_t units, uint32_t nz) {
+    return nz > 1 ? units - units / nz + 1u : 0u;
+}
+
+/* What a split's memory costs a call on its own: it is allocated in stream
+ * order, but the pool keeps none of it over a synchronisation, and the call
+ * after one pays 10 - 60 us for it by its size (a process's first, or a larger
+ * one than any before, 100 - 500). Up to one tile per CU a split fills the chip
+ * and gains more; past it the gain must cover most of this, or a call on its own
+ * runs slower than unsplit (2560 x 2048 Q4_K, 1,020 tokens, split without this:
+ * 209 us in a run of calls but 305 each on its own, against 228 and 239
+ * unsplit), and the memory stays below a thousandth of the card's. */
+#define GEMM_PAST_BYTES ((uint64_t)256 << 20)
+
+static double gemm_past_ns(uint64_t bytes) {
+    const double ns = 12000.0 + 0.45e-3 * (double)bytes;
+    return ns < 30000.0 ? ns : 30000.0;
+}
+
 /* Nanoseconds per column step and SIMD with w waves on it, measured on MI355X
  * (Q4_K 512 .. 9728 rows x 2048 / 2560 columns, 512 and 2047 tokens), by kw
  * (1, 2, 4) and w. The bound is 28.7 at 2 or 4 waves, 34 at 3, 43.7 at 1;
@@ -46,14 +67,18 @@ static const double gemm_step_ns[3][5] = {{0.0, 54.0, 37.8, 37.3, 33.0},
  * waves per SIMD it leaves; a split costs the fold's traffic (each unit sum
  * past the first split written and read, about 4.5 TB/s) and its launch.
  * cap: most splits. unit_steps: MFMAs of a super-block and wave (256, or 64 a
- * 16-token group in the kernels for few tokens). */
+ * 16-token group in the kernels for few tokens). past: the whole product has
+ * more than one tile per CU, so a split must also gain what its memory costs a
+ * call on its own, and keep to GEMM_PAST_BYTES of it. */
 static gemm_split gemm_plan(uint64_t tiles, uint32_t units, uint64_t outputs, uint32_t cus,
-                            uint32_t max_kw, uint32_t cap, double unit_steps) {
+                            uint32_t max_kw, uint32_t cap, double unit_steps, int past) {
     gemm_split best = {1, 1, 0.0};
     for (uint32_t kw = 1, i = 0; kw <= max_kw && kw <= units; kw *= 2u, i++) {
         const uint64_t slots = (uint64_t)cus * (4u / kw);
         for (uint32_t nz = 1; nz <= cap && nz <= units; nz++) {
             if (nz > 1 && tiles * (nz - 1u) >= slots) break;
+            const uint64_t bytes = 4u * outputs * gemm_slots(units, nz);
+            if (past && bytes > GEMM_PAST_BYTES) continue;
             const uint32_t per = (units + nz - 1u) / nz;
             const double steps = unit_steps * (double)((per + kw - 1u) / kw);
             uint64_t left = tiles * nz;
@@ -65,7 +90,7 @@ static gemm_split gemm_plan(uint64_t tiles, uint32_t units, uint64_t outputs, ui
                 ns += steps * (double)w * gemm_step_ns[i][w];
             }
             if (nz > 1)
-                ns += 4000.0 + (double)outputs * 8.0 * (double)(units - units / nz + 1u) / 4500.0;
+                ns += 4000.0 + 2.0 * (double)bytes / 4500.0 + (past ? gemm_past_ns(bytes) : 0.0);
             if (best.ns == 0.0 || ns < best.ns) {
                 best.ns = ns;
                 best.kw = kw;
@@ -84,17 +109,18 @@ static uint32_t gemm_few(size_t tokens) {
     return tokens <= 32 && env_long("MYNAH_GEMM_FEW", 1) ? (uint32_t)(tokens + 15) / 16 : 0u;
 }
 
+/* split: 0 keeps nz at 1; past: as gemm_plan's. */
 static gemm_split gemm_split_of(const mynah_device *d, int type, int ord, size_t rows, size_t cols,
-                                size_t tokens) {
+                                size_t tokens, int split, int past) {
     const uint32_t few = gemm_few(tokens);
     const uint64_t tiles = (uint64_t)((rows + 63) / 64) * ((tokens + 63) / 64);
     const double steps = few ? 64.0 * few : 256.0;
     const uint32_t units = (uint32_t)(cols / 256);
     /* The Q8_0 matvec order has no unit sums to split by. */
     const int whole = ord == 1 && type == MYNAH_Q8_0;
-    const long cap = whole ? 1 : env_long("MYNAH_GEMM_SPLIT", 64);
+    const long cap = whole || !split ? 1 : env_long("MYNAH_GEMM_SPLIT", 64);
     return gemm_plan(tiles, units, (uint64_t)rows * tokens, (uint32_t)d->cus,
-                     few || whole ? 1u : 4u, cap > 1 ? (uint32_t)cap : 1u, steps);
+                     few || whole ? 1u : 4u, cap > 1 ? (uint32_t)cap : 1u, steps, past);
 }
 
 /* The exact GEMM with its products on MFMA (gemm_mfma.hip): the default;
@@ -128,8 +154,8 @@ static int gemm_mfma_part(mynah_device *d, int type, int ord, const void *w, siz
     void *args[] = {&w, &x, &y, &r32, &c32, &t32, &rb32, &res, &part};
     int rc = mynah_launch3(d, kernel, gx, gy, nz, block, 0, stream, args);
     if (rc == 0 && nz > 1) {
-        uint32_t u32 = units, first = units / nz;   /* the units of split 0 */
-        void *fargs[] = {&part, &res, &y, &r32, &t32, &first, &u32};
+        uint32_t slots = gemm_slots(units, nz);
+        void *fargs[] = {&part, &res, &y, &r32, &t32, &slots};
         rc = mynah_launch(d, MYNAH_K_GEMM_FOLD, (unsigned)((rows * tokens + 255) / 256), 1, 256, 0,
                           stream, fargs);
     }
@@ -142,39 +168,48 @@ static int gemm_mfma_part(mynah_device *d, int type, int ord, const void *w, siz
  * for few tokens. Every output is the same sum either way. 9728 x 2560 Q4_K, 65
  * tokens: 145 -> 97 us; 201: 246 -> 216; 2560 x 9728 Q6_K, 201: 263 -> 232;
  * 6144 x 2048 Q4_K, 130: 105 -> 90. Not for the Q8_0 matvec order, which cannot
- * split the second product (4096 x 2048, 270 tokens: 166 -> 169). */
+ * split the second product (4096 x 2048, 270 tokens: 166 -> 169).
+ *
+ * Without the memory for a split's sums the product runs unsplit. */
 static int gemm_mfma_launch(mynah_device *d, int type, int ord, const void *w, size_t rows,
                             size_t cols, size_t rb, const float *x, float *y, size_t tokens,
                             const float *res, hipStream_t stream) {
     const long kw = env_long("MYNAH_GEMM_KW", 0);
     const int whole = ord == 1 && type == MYNAH_Q8_0;
-    size_t head = tokens, last = tokens % 64;
-    gemm_split ph = gemm_split_of(d, type, ord, rows, cols, tokens), pl = {1, 1, 0.0};
-    if (!whole && last > 0 && last < tokens && gemm_few(last)) {
-        const gemm_split a = gemm_split_of(d, type, ord, rows, cols, tokens - last);
-        pl = gemm_split_of(d, type, ord, rows, cols, last);
-        if (a.ns + pl.ns + 8000.0 < ph.ns) {
-            head = tokens - last;
-            ph = a;
+    const uint32_t units = (uint32_t)(cols / 256);
+    const int past = (uint64_t)((rows + 63) / 64) * ((tokens + 63) / 64) > (uint64_t)d->cus;
+    int split = 1;
+    size_t head, last, bytes;
+    gemm_split ph, pl;
+    float *part;
+    for (;; split = 0) {
+        head = tokens;
+        last = tokens % 64;
+        ph = gemm_split_of(d, type, ord, rows, cols, tokens, split, past);
+        pl = (gemm_split){1, 1, 0.0};
+        if (!whole && last > 0 && last < tokens && gemm_few(last)) {
+            const gemm_split a =
+                gemm_split_of(d, type, ord, rows, cols, tokens - last, split, past);
+            pl = gemm_split_of(d, type, ord, rows, cols, last, split, past);
+            if (a.ns + pl.ns + 8000.0 < ph.ns) {
+                head = tokens - last;
+                ph = a;
+            }
         }
-    }
-    if (!whole && !gemm_few(head) && (kw == 1 || kw == 2 || kw == 4))
-        ph.kw = (uint32_t)kw;
-    size_t n = ph.nz > 1 ? rows * head : 0;
-    if (head < tokens && pl.nz > 1 && rows * last > n) n = rows * last;
-    const size_t bytes = cols / 256 * n * sizeof(float);
-    float *part = NULL;
-    hipError_t e = bytes ? hipMallocAsync((void **)&part, bytes, stream) : hipSuccess;
-    if (e != hipSuccess) {
-        mynah_set_error("hipMallocAsync(split-K partials, %zu bytes): %s", bytes,
-                        hipGetErrorString(e));
-        return -1;
+        if (!whole && !gemm_few(head) && (kw == 1 || kw == 2 || kw == 4)) ph.kw = (uint32_t)kw;
+        size_t n = gemm_slots(units, ph.nz) * (rows * head);
+        if (head < tokens && gemm_slots(units, pl.nz) * (rows * last) > n)
+            n = gemm_slots(units, pl.nz) * (rows * last);
+        bytes = n * sizeof(float);
+        part = NULL;
+        if (bytes == 0 || hipMallocAsync((void **)&part, bytes, stream) == hipSuccess) break;
+        (void)hipGetLastError();
     }
     int rc = gemm_mfma_part(d, type, ord, w, rows, cols, rb, x, y, head, res, ph, part, stream);
     if (rc == 0 && head < tokens)
         rc = gemm_mfma_part(d, type, ord, w, rows, cols, rb, x + head * cols, y + head * rows, last,
                             res ? res + head * rows : NULL, pl, part, stream);
-    e = bytes ? hipFreeAsync(part, stream) : hipSuccess;
+    const hipError_t e = bytes ? hipFreeAsync(part, stream) : hipSuccess;
     if (rc == 0 && e != hipSuccess) {
         mynah_set_error("hipFreeAsync(split-K partials): %s", hipGetErrorString(e));
         return -1;

@@ -33,7 +33,7 @@ def test_few_tokens(M, monkeypatch, qtype, mv, rows, units, tokens):  # noqa: F8
 
 
 @pytest.mark.parametrize("rows,cols,tokens", [(4096, 2560, 65), (4095, 2560, 80), (2048, 2048, 270),
-                                              (2560, 9728, 96)])
+                                              (2560, 9728, 96), (9728, 2816, 216)])
 @pytest.mark.parametrize("mv", [False, True])
 @pytest.mark.parametrize("qtype", [12, 13, 14, 8])
 def test_few_tokens_past_the_last_tile(M, monkeypatch, qtype, mv, rows, cols, tokens):  # noqa: F811
