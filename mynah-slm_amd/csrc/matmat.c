@@ -37,17 +37,17 @@ static uint32_t gemm_slots(uint32_t units, uint32_t nz) {
 
 /* What a split's memory costs a call on its own: it is allocated in stream
  * order, but the pool keeps none of it over a synchronisation, and the call
- * after one pays 10 - 60 us for it by its size (a process's first, or a larger
- * one than any before, 100 - 500). Up to one tile per CU a split fills the chip
- * and gains more; past it the gain must cover most of this, or a call on its own
- * runs slower than unsplit (2560 x 2048 Q4_K, 1,020 tokens, split without this:
- * 209 us in a run of calls but 305 each on its own, against 228 and 239
- * unsplit), and the memory stays below a thousandth of the card's. */
+ * after one pays about 20 us for up to 64 MiB of it and 40 - 85 for more (a
+ * process's first, or a larger one than any before, 100 - 500). Up to one tile
+ * per CU a split fills the chip and gains more. Past it the gain must cover most
+ * of this, the line between runs of calls and calls on their own (2560 x 2048
+ * Q4_K, 1,020 tokens, split without this: 209 us in a run of calls but 305 each
+ * on its own, against 228 and 239 unsplit), and the memory stays below a
+ * thousandth of the card's. */
 #define GEMM_PAST_BYTES ((uint64_t)256 << 20)
 
 static double gemm_past_ns(uint64_t bytes) {
-    const double ns = 12000.0 + 0.45e-3 * (double)bytes;
-    return ns < 30000.0 ? ns : 30000.0;
+    return bytes <= ((uint64_t)64 << 20) ? 15000.0 : 30000.0;
 }
 
 /* Nanoseconds per column step and SIMD with w waves on it, measured on MI355X
@@ -68,8 +68,8 @@ static const double gemm_step_ns[3][5] = {{0.0, 54.0, 37.8, 37.3, 33.0},
  * past the first split written and read, about 4.5 TB/s) and its launch.
  * cap: most splits. unit_steps: MFMAs of a super-block and wave (256, or 64 a
  * 16-token group in the kernels for few tokens). past: the whole product has
- * more than one tile per CU, so a split must also gain what its memory costs a
- * call on its own, and keep to GEMM_PAST_BYTES of it. */
+ * more than one tile per CU, so a split must also gain gemm_past_ns and keep to
+ * GEMM_PAST_BYTES of memory. */
 static gemm_split gemm_plan(uint64_t tiles, uint32_t units, uint64_t outputs, uint32_t cus,
                             uint32_t max_kw, uint32_t cap, double unit_steps, int past) {
     gemm_split best = {1, 1, 0.0};
