@@ -393,7 +393,7 @@ MYNAH_DEV void gf_stage_few(gf_f32x16 &s, gf_f32x16 &acc, float *v, const uint8_
     auto product = [&](const float b, int i) __attribute__((always_inline)) {
         return __builtin_amdgcn_mfma_f32_16x16x1f32(a[i / G], b, zero, 0, 0, 0);
     };
-    constexpr int N = 16 * G, AHEAD = 4;
+    constexpr int N = 16 * G, AHEAD = FOLD32 && G == 1 ? 2 : MIXED && G == 2 ? 3 : 4;
     float xb[AHEAD];
 #pragma unroll
     for (int i = 0; i < AHEAD; i++) xb[i] = fetch(i);
@@ -565,9 +565,14 @@ GEMM_MFMA_ENTRIES(mynah_q4k_gemm_mv_mfma, GfQ4K, 1, 12)
 GEMM_MFMA_ENTRIES(mynah_q5k_gemm_mv_mfma, GfQ5K, 1, 13)
 GEMM_MFMA_ENTRY(mynah_q80_gemm_mv_mfma1, GfQ80, 1, 8, 1)
 
-// At most 16 G tokens: grid (ceil(rows / 64), 1, Z), block 256.
+// At most 16 G tokens: grid (ceil(rows / 64), 1, Z), block 256. Four waves a
+// SIMD like the full tile's, which the host's plan counts on: left at 129 - 132
+// registers, four of them held three (17 - 32 tokens: 6874 x 8448 Q4_K, matvec
+// order 110 -> 95 us, 10434 x 4096 Q5_K 88 -> 78, 7229 x 8448 Q6_K 115 -> 100).
+// x is read fewer steps ahead where the registers would not hold it; the Q6_K
+// form for 32 tokens spills one.
 #define GEMM_FEW_ENTRY(name, RAW, ORD, FMT, G)                                                \
-    extern "C" __global__ void __launch_bounds__(256, 2)                                       \
+    extern "C" __global__ void __launch_bounds__(256, 4)                                       \
         name(const uint8_t *__restrict__ w, const float *__restrict__ x, float *y,             \
              uint32_t rows, uint32_t cols, uint32_t tokens, uint32_t row_bytes,                \
              const float *res, float *part) {                                                  \
