@@ -121,13 +121,16 @@ static const int8_tile int8_tiles[4] = {{32, 32, 4, 5, 1.1, 0.22},
 /* The tile of least estimated time: rounds of resident workgroups, the last
  * with as many per CU as are left. The kernels address a tile's rows of
  * weights and of activations in 32 bits: rows too long for the larger tiles
- * take the smallest. MYNAH_INT8_TILE=0..3 forces one. */
+ * take the smallest. MYNAH_INT8_TILE=0..3 forces one of those that the rows'
+ * length allows. */
 static int int8_plan(size_t rows, size_t tokens, size_t cols, uint32_t cus) {
+    const int tiles = cols < ((size_t)1 << 24) ? 4 : 1;
     const char *env = getenv("MYNAH_INT8_TILE");
-    if (env != NULL && env[0] >= '0' && env[0] <= '3' && env[1] == '\0') return env[0] - '0';
+    if (env != NULL && env[0] >= '0' && env[0] < '0' + tiles && env[1] == '\0')
+        return env[0] - '0';
     int best = 0;
     double best_t = 0.0;
-    for (int i = 0; i < 4 && (i == 0 || cols < ((size_t)1 << 24)); i++) {
+    for (int i = 0; i < tiles; i++) {
         const int8_tile *t = &int8_tiles[i];
         const uint64_t wgs = (uint64_t)((rows + t->rows - 1) / t->rows) *
                              (uint64_t)((tokens + t->toks - 1) / t->toks);

@@ -1,6 +1,6 @@
-"""The host side of the exact batched products (csrc/matmat.c), on the CPU:
-its launches and its workspace, recorded by oracle/plan_pin.c. For products on
-both sides of one tile per CU, in both orders and every type:
+"""The host side of the batched products (csrc/matmat.c, csrc/int8.c), on the
+CPU: its launches and its workspace, recorded by oracle/plan_pin.c. For exact
+products on both sides of one tile per CU, in both orders and every type:
 
 * the launches cover every token once, in order, by the tiles of the kernel
   that takes them;
@@ -8,6 +8,9 @@ both sides of one tile per CU, in both orders and every type:
   per later super-block) fit the workspace, which holds nothing else, and a
   product of more than one tile per CU keeps to 256 MiB of it;
 * where the workspace cannot be had, the same product runs unsplit.
+
+The int8 lane's larger tiles address their rows in 32 bits: rows too long for
+them take the smallest tile, also where the environment names another.
 """
 from __future__ import annotations
 
@@ -102,3 +105,17 @@ def test_runs_unsplit_without_the_workspace(lane, qtype):
         assert sum(x.tokens for x in launches) == tokens
         tried += allocs
     assert tried or (lane == "matvec" and qtype == Q8_0)
+
+
+@pytest.mark.parametrize("tile", [None, "0", "1", "2", "3"])
+@pytest.mark.parametrize("qtype", [Q4_K, Q5_K])
+def test_int8_tiles_by_row_length(monkeypatch, qtype, tile):
+    monkeypatch.delenv("MYNAH_INT8_TILE", raising=False)
+    if tile is not None:
+        monkeypatch.setenv("MYNAH_INT8_TILE", tile)
+    names = [b"32x32", b"64x64", b"96x128", b"128x128"]
+    quant, gemm = plan("int8", qtype, 9728, 4096, 2048)[0]
+    assert gemm.kernel.split(b"_")[-1] in ([names[int(tile)]] if tile else names)
+    for cols in (1 << 24, 1 << 26):
+        quant, gemm = plan("int8", qtype, 256, cols, 128)[0]
+        assert gemm.kernel.endswith(b"32x32") and (gemm.gx, gemm.gy) == (8, 4)
