@@ -105,10 +105,15 @@ int mynah_q8_quantize_launch(mynah_device *d, const float *x, size_t tokens, siz
     return mynah_launch(d, MYNAH_K_Q8_QUANTIZE, (units + 3u) / 4u, 1, 256, 0, stream, args);
 }
 
-/* The batched kernels' workgroup tiles, in the kernel ids' order: how many fit
- * a CU (LDS), and the microseconds one super-block takes with k of them there,
- * t0 + k t1 (measured on MI355X at 512 and 2047 tokens; a lone small tile waits
- * for its copies, full CUs issue). */
+/* The batched kernels' workgroup tiles, in the kernel ids' order: how many the
+ * plan takes a CU to hold, and the microseconds one super-block takes with k of
+ * them there, t0 + k t1 (measured on MI355X at 512 and 2047 tokens; a lone small
+ * tile waits for its copies, full CUs issue). Q4_K's small tile fits five times
+ * (LDS), Q5_K's four (33,024 bytes, 100 registers); both are planned as five: a
+ * fifth workgroup starts as soon as one of four ends, not a round later, and
+ * counted as four the plan took larger tiles too early (6016 x 4608 Q5_K, 182
+ * tokens: 58 -> 67 us; 1984 x 5120, 593 tokens: 65 -> 75; of 100 drawn products
+ * of 900 - 2,200 small tiles none gained more than the runs differ). */
 typedef struct {
     uint32_t rows, toks, waves, per_cu;
     double t0, t1;
