@@ -1026,12 +1026,14 @@ static int enqueue_prefill_chunk(mynah_qwen3 *s, mynah_device *d, hipStream_t st
             uint32_t tt = T;
             /* Four (32 queries, head) pairs per workgroup, and the most
              * positions, 128 at most, that still make SCORES_WGS workgroups
-             * (the queries are loaded once per workgroup). */
+             * (the queries are loaded once per workgroup).
+             * MYNAH_PREFILL_SPAN forces them, as a multiple of 32. */
             const uint32_t zs = (group * ((T + 31) / 32) + 3) / 4;
-            uint32_t span = (uint32_t)env_or("MYNAH_PREFILL_SPAN", 128) & ~31u;
-            if (span < 32) span = 32;
-            while (span > 32 && c->n_kv_heads * zs * ((p0 + T + span - 1) / span) < SCORES_WGS)
-                span = (span / 2 + 31) & ~31u;
+            const long forced = env_or("MYNAH_PREFILL_SPAN", 0);
+            uint32_t span = forced >= 32 && forced <= 65536 ? (uint32_t)forced & ~31u : 128u;
+            while (forced <= 0 && span > 32 &&
+                   c->n_kv_heads * zs * ((p0 + T + span - 1) / span) < SCORES_WGS)
+                span /= 2;
             void *args[] = {&qn, &kc, &sc, &p0, &tt, &sstride, &kvd, &grp, &scale, &span};
             rc = mynah_launch3(d, MYNAH_K_PREFILL_SCORES, c->n_kv_heads, (p0 + T + span - 1) / span,
                                zs, 256, 0, st, args);
