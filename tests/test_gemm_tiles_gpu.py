@@ -21,7 +21,7 @@ def M():
 
 
 def product(M, monkeypatch, env, mv, qtype, w, rows, cols, x, tokens, res):
-    for k in ("MYNAH_GEMM_MFMA", "MYNAH_GEMM_SPLIT", "MYNAH_GEMM_KW"):
+    for k in ("MYNAH_GEMM_MFMA", "MYNAH_GEMM_SPLIT", "MYNAH_GEMM_KW", "MYNAH_GEMM_FEW"):
         monkeypatch.delenv(k, raising=False)
     for k, v in env.items():
         monkeypatch.setenv(k, v)
@@ -61,9 +61,12 @@ def test_tiles_and_wave_groups(M, monkeypatch, qtype, mv, rows, units, tokens):
     res = M.synth_normal(tokens, tokens * rows) if mv else None
     ref = product(M, monkeypatch, {"MYNAH_GEMM_MFMA": "0"}, mv, qtype, w, rows, cols, x, tokens,
                   res)
-    # Few tiles: the plan splits over super-blocks unless told not to.
-    for env in ({}, {"MYNAH_GEMM_SPLIT": "0"},
-                *({"MYNAH_GEMM_KW": k, "MYNAH_GEMM_SPLIT": s} for k in "124" for s in "03")):
+    # Few tiles: the plan splits over super-blocks unless told not to. The full
+    # tile also where at most 32 tokens would take kernels of their own
+    # (MYNAH_GEMM_FEW=0).
+    for env in ({}, {"MYNAH_GEMM_SPLIT": "0"}, {"MYNAH_GEMM_FEW": "0"},
+                *({"MYNAH_GEMM_KW": k, "MYNAH_GEMM_SPLIT": s, "MYNAH_GEMM_FEW": "0"}
+                  for k in "124" for s in "03")):
         got = product(M, monkeypatch, env, mv, qtype, w, rows, cols, x, tokens, res)
         assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), env
 
@@ -82,5 +85,5 @@ def test_any_block_and_non_finite_activations(M, monkeypatch, qtype, mv):
     ref = product(M, monkeypatch, {"MYNAH_GEMM_MFMA": "0"}, mv, qtype, w, rows, cols, x, tokens,
                   None)
     for k in "124":
-        env = {"MYNAH_GEMM_KW": k}
+        env = {"MYNAH_GEMM_KW": k, "MYNAH_GEMM_FEW": "0"}
         assert same(product(M, monkeypatch, env, mv, qtype, w, rows, cols, x, tokens, None), ref)

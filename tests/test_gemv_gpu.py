@@ -270,7 +270,7 @@ def test_mfma_gemm_equals_valu_gemm(M, qtype, mv):
     64-token tile. The products of v_mfma_f32_16x16x1_4b_f32 with a zero
     accumulator are v_mul_f32's (a -0 comes out +0, which no sum here can
     see)."""
-    keys = ("MYNAH_GEMM_MFMA", "MYNAH_GEMM_SPLIT", "MYNAH_GEMM_WGS_PER_CU")
+    keys = ("MYNAH_GEMM_MFMA", "MYNAH_GEMM_SPLIT")
     saved = {k: os.environ.get(k) for k in keys}
 
     def run(env, rows, cols, tokens, res):
