@@ -265,6 +265,15 @@ int   mynah_hip_valu_add_rate(uint32_t iters, float *ns_per_instr, uint32_t *sim
  * buffers: a, b 64 * waves floats, the rest 1024 * waves. */
 int   mynah_hip_mfma_probe(const float *a, const float *b, const float *c, float *prod,
                            float *acc, float *mul, float *fused, uint32_t waves, void *stream);
+/* The chain of the batched prefill's matrix-core instruction (no reference
+ * counterpart; a test hook): per wave w < waves, a[64 w + 16 k + i] is row i and
+ * b[64 w + 16 k + j] column j at position k < 4, c the accumulator; acc (the
+ * instruction) and fused (c, then fmaf of the four products in k order) get
+ * 256 w + 4 l + e for row 4 (l / 16) + e, column l % 16, as c is laid out.
+ * Device buffers: a, b 64 * waves floats, the rest 256 * waves, c 16-byte
+ * aligned. */
+int   mynah_hip_mfma_chain_probe(const float *a, const float *b, const float *c, float *acc,
+                                 float *fused, uint32_t waves, void *stream);
 void *mynah_hip_stream(void);           /* the library's own stream */
 
 /* y[i] = expf(x[i]) for i < n with the bits of the reference's C library

@@ -2100,3 +2100,29 @@ MYNAH_DEV void prefill_pv(const float *__restrict__ v_layer, const float *__rest
     }
 PV_KERNEL(128, 3)      // 63 positions x 16 heads: 8.4 us, 2,047 x 32: 153 us
 PV_KERNEL(32, 4)       // 63 positions x 16 heads: 5.0 us, 2,047 x 32: 175 us
+
+// Test hook for the chain property that the two kernels above rest on (no
+// reference counterpart). Per workgroup (one wave) 16 x 4 values of a, 4 x 16
+// of b and 16 x 16 of c: acc = v_mfma_f32_16x16x4_f32 of them, fused = c and
+// the four products of each output taken in k order with fmaf. a of row i and
+// position k at 64 blockIdx + 16 k + i, b likewise by column; c, acc and fused
+// of row 4 (l / 16) + e, column l % 16 at 256 blockIdx + 4 l + e.
+extern "C" __global__ void __launch_bounds__(64)
+mynah_mfma_chain_probe(const float *__restrict__ a, const float *__restrict__ b,
+                       const float *__restrict__ c, float *__restrict__ acc,
+                       float *__restrict__ fused) {
+    const uint32_t l = threadIdx.x;
+    const size_t base = 64u * (size_t)blockIdx.x, out = 4u * (base + l);
+    const v4f cv = *(const v4f *)(c + out);
+    const v4f d = __builtin_amdgcn_mfma_f32_16x16x4f32(a[base + l], b[base + l], cv, 0, 0, 0);
+#pragma unroll
+    for (uint32_t e = 0; e < 4; e++) {
+        float f = cv[e];
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++)
+            f = __builtin_fmaf(a[base + 16u * k + 4u * (l / 16u) + e], b[base + 16u * k + l % 16u],
+                               f);
+        acc[out + e] = d[e];
+        fused[out + e] = f;
+    }
+}

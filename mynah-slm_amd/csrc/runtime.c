@@ -1234,6 +1234,20 @@ int mynah_hip_mfma_probe(const float *a, const float *b, const float *c, float *
                         mynah_stream_or_default(d, stream), args);
 }
 
+int mynah_hip_mfma_chain_probe(const float *a, const float *b, const float *c, float *acc,
+                               float *fused, uint32_t waves, void *stream) {
+    mynah_device *d = mynah_dev();
+    if (d == NULL) return -1;
+    if (a == NULL || b == NULL || c == NULL || acc == NULL || fused == NULL || waves == 0 ||
+        waves > 65535u || (((uintptr_t)c) & 15u) != 0) {
+        mynah_set_error("mfma chain probe: null or misaligned buffer, or waves outside 1..65535");
+        return -1;
+    }
+    void *args[] = {&a, &b, &c, &acc, &fused};
+    return mynah_launch(d, MYNAH_K_MFMA_CHAIN_PROBE, waves, 1, 64, 0,
+                        mynah_stream_or_default(d, stream), args);
+}
+
 int mynah_hip_valu_add_rate(uint32_t iters, float *ns_per_instr, uint32_t *simds) {
     mynah_device *d = mynah_dev();
     if (d == NULL) return -1;

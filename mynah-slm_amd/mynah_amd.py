@@ -113,6 +113,7 @@ def _load() -> C.CDLL:
         "mynah_hip_event_destroy": (C.c_int, [_P]),
         "mynah_hip_copy_dev": (C.c_int, [_P, _P, _SZ, _P]),
         "mynah_hip_read_dev": (C.c_int, [_P, _SZ, _P, _P]),
+        "mynah_hip_mfma_chain_probe": (C.c_int, [_P, _P, _P, _P, _P, C.c_uint32, _P]),
         "mynah_hip_mfma_probe": (C.c_int, [_P, _P, _P, _P, _P, _P, _P, C.c_uint32, _P]),
         "mynah_hip_valu_add_rate": (C.c_int, [C.c_uint32, C.POINTER(C.c_float),
                                               C.POINTER(C.c_uint32)]),
