@@ -20,7 +20,9 @@ MYNAH_DEV float f16_to_f32(uint32_t bits16) {
 
 // Byte K of a dword as float: one v_cvt_f32_ubyte{K}. Written as inline asm
 // because the compiler otherwise folds a preceding nibble mask into a v_bfe
-// and converts byte 0, which costs an extra instruction per weight.
+// and converts byte 0, which costs an extra instruction per weight. Not for
+// kernels with MFMA: inline asm in one makes the compiler keep MFMA results in
+// the accumulation registers, which costs a v_accvgpr_read per result.
 template <int K>
 MYNAH_DEV float ubyte_f(uint32_t v) {
     float r;
@@ -29,16 +31,6 @@ MYNAH_DEV float ubyte_f(uint32_t v) {
     else if (K == 2) asm("v_cvt_f32_ubyte2 %0, %1" : "=v"(r) : "v"(v));
     else asm("v_cvt_f32_ubyte3 %0, %1" : "=v"(r) : "v"(v));
     return r;
-}
-
-// ubyte_f (ASM) or the plain conversion (the backend picks the instruction).
-// Kernels with MFMA take the plain form: inline asm in a kernel makes the
-// compiler keep MFMA results in the accumulation registers, which costs a
-// v_accvgpr_read per result before it can be used.
-template <bool ASM, int K>
-MYNAH_DEV float ubyte_sel(uint32_t v) {
-    if constexpr (ASM) return ubyte_f<K>(v);
-    else return (float)((v >> (8 * K)) & 0xffu);
 }
 
 // Byte k of a dword as float (plain C; the backend picks the conversion).

@@ -62,8 +62,8 @@ def test_the_instruction_is_a_chain_of_fmaf():
     # fmaf in the reverse order (through doubles: all but its double roundings)
     # and products rounded on their own give other sums.
     x, y = products(a, b)
-    back, apart = c.astype(np.float64), c.copy()
     with np.errstate(all="ignore"):
+        back, apart = c.astype(np.float64), c.copy()
         for k in range(4):
             back = (x[3 - k].astype(np.float64) * y[3 - k] + back).astype(np.float32) \
                 .astype(np.float64)
