@@ -777,7 +777,7 @@ int mynah_dequant_launch(mynah_device *d, int type, const void *w, size_t rows, 
         return -1;
     }
     uint64_t quads = (uint64_t)rows * (cols / 4);
-    const uint64_t grid = (quads + 256u * 4u - 1u) / (256u * 4u);   /* DQ_STEP = 4 */
+    const uint64_t per_wg = 256u * MYNAH_DQ_STEP, grid = (quads + per_wg - 1u) / per_wg;
     if (grid > 0x7fffffffu) {
         mynah_set_error("dequant too large");
         return -1;

@@ -129,10 +129,9 @@ enum {
 
 #define MYNAH_MAX_DEVICES 16
 
-/* Positions per workgroup of the generic split attention kernel (decode.hip
- * AS_CH); the kernels for 2 and 4 query heads per key head take 32, 64 or
- * 128, chosen by the context length. */
-/* Dimensions per workgroup of the exact attention's PV kernel (= PV_SW in
+/* Quads of values per thread of the dequantiser (= DQ_STEP in dequant.hip). */
+#define MYNAH_DQ_STEP 4u
+/* Dimensions per workgroup of the exact attention's PV kernel (= DPV_SW in
  * decode.hip). */
 #define MYNAH_PV_SW 16
 /* Most positions of the one-launch exact attention (= ASH_N in decode.hip). */
@@ -141,6 +140,9 @@ enum {
 #ifndef MYNAH_PV_LW
 #define MYNAH_PV_LW 4
 #endif
+/* Positions per workgroup of the generic split attention kernel (= AS_CH in
+ * common.hip.h); the kernels for 2 and 4 query heads per key head take 32, 64 or
+ * 128, chosen by the context length. */
 #define MYNAH_AS_CH 32
 /* Most chunks mynah_attn_combine1 (one wave per query head) takes. */
 #define MYNAH_AC1_MAX 32

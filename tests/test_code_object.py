@@ -1,6 +1,7 @@
 """What the host's plans assume of the compiled kernels (the registers and LDS
 in the code object's metadata), on the CPU: csrc/matmat.c counts on four waves
-per SIMD of every exact GEMM kernel on the matrix cores.
+per SIMD of every exact GEMM kernel on the matrix cores; and the sizes that a
+kernel and the host code launching it both state.
 """
 from __future__ import annotations
 
@@ -46,3 +47,17 @@ def test_exact_gemm_kernels_hold_four_waves_per_simd(kernels):
         k = kernels[n]
         assert workgroups_per_cu(k) * (k["max_flat_workgroup_size"] // 64) >= 16, (n, k)
         assert k["vgpr_spill_count"] <= 1, (n, k)
+
+
+@pytest.mark.parametrize("host,source,kernel", [
+    ("MYNAH_DQ_STEP", "dequant.hip", "DQ_STEP"), ("MYNAH_PV_SW", "decode.hip", "DPV_SW"),
+    ("MYNAH_ATTN_SHORT_N", "decode.hip", "ASH_N"), ("MYNAH_AS_CH", "common.hip.h", "AS_CH")])
+def test_sizes_stated_twice_agree(host, source, kernel):
+    def value(path, name):
+        with open(os.path.join(ROOT, "mynah-slm_amd", "csrc", path)) as f:
+            text = f.read()
+        expr = re.search(rf"#define {name} ([^\n/]+)", text).group(1).strip()
+        while re.search(r"[A-Z_]{3,}", expr):
+            expr = re.sub(r"[A-Z_]{3,}", lambda m: str(value(path, m.group(0))), expr)
+        return eval(re.sub(r"(\d)u\b", r"\1", expr))      # noqa: S307 (the source's own constant)
+    assert value("runtime_internal.h", host) == value(source, kernel)
