@@ -33,7 +33,7 @@ greedy steps on Qwen3-4B), `qwen3_4b_gemv_gbs` (each Qwen3-4B GEMV class),
 read-only stream moving the same HBM bytes per launch: what any kernel
 launched back to back reaches at that size) and `valu` (the time per wave64
 f32 add with every SIMD issuing adds only, and the exact GEMM's ceiling that
-follows from one add per product).
+follows from one add per product beside the MFMA that makes the products).
 
 Usage: python bench.py [--gpus 1] [--steps K] [--warmup W]
 """
@@ -401,12 +401,14 @@ def gpu_prefill_gemm(M, CF, reps: int = 20, int8: bool = False):
                     "peak_top_s_int8": PEAK_INT8_TOPS,
                     "frac_of_int8_peak": round(q4_flop / q4_ms / 1e9 / PEAK_INT8_TOPS, 4),
                     "note": "integer dots on v_mfma_i32_16x16x32_i8; the reference's f32 "
-                            "epilogue (a convert and two fma per dot) bounds it on the VALU"})
+                            "epilogue on the VALU (a subtraction and two fma per dot, in the "
+                            "128 x 128 tile one) and the MFMAs do not overlap: issue bounds it"})
     else:
         res.update({"peak_tflop_s_fp32": PEAK_FP32_TFLOPS,
                     "frac_of_fp32_peak": round(tot_flop / tot_ms / 1e9 / PEAK_FP32_TFLOPS, 4),
                     "note": "one mul and one add per product (the reference's roundings): the "
-                            "non-packed VALU issue rate bounds this order near 40 TFLOP/s"})
+                            "muls on the matrix cores and the adds on the VALU do not overlap; "
+                            "valu.exact_gemm_ceiling_tflop_s is what that leaves this order"})
     return res
 
 
@@ -720,12 +722,18 @@ def pmc_probe(M, CF, launches: int = 8) -> None:
         f"4 copies of {nbytes} bytes (mynah_copy16)")
 
 
+# Nanoseconds of its SIMD that the exact GEMM's MFMA takes (1,024 products), at
+# any number of waves (profiles/issue_rates.md).
+EXACT_MFMA_NS = 13.55
+
+
 def valu_yardstick(M, prefill) -> dict:
-    """The exact orders pay one non-packed v_add_f32 per product: the time per
-    wave64 add (every SIMD issuing only adds) bounds the exact GEMM at
-    2 flops x 64 lanes / t per SIMD. Measured twice, the faster kept."""
+    """The exact orders pay one non-packed v_add_f32 per product, 16 wave64 adds
+    per MFMA of the exact GEMM, and the two do not overlap: the time per add
+    (every SIMD issuing only adds) and the MFMA's bound the exact GEMM. Measured
+    twice, the faster kept."""
     ns, simds = min(M.valu_add_rate() for _ in range(2))
-    ceiling = 2.0 * 64.0 / (ns * 1e-9) * simds / 1e12
+    ceiling = 2.0 * 1024.0 / ((16.0 * ns + EXACT_MFMA_NS) * 1e-9) * simds / 1e12
     out = {"f32_add_ns_per_wave64_per_simd": round(ns, 4), "simds": simds,
            "exact_gemm_ceiling_tflop_s": round(ceiling, 1)}
     if prefill is not None:
