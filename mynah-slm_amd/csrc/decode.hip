@@ -1784,7 +1784,7 @@ mynah_prefill_rope(float *__restrict__ q, float *__restrict__ k_layer,
 // different banks. Grid (n_kv_heads, ceil((p0 + T) / span), ceil(group ceil(T /
 // PS_Q) / 4)), block 256; the host takes the longest span that still fills the
 // chip.
-// What bounds it: the MFMAs, 32 of 13.6 ns per 256 scores on a SIMD, and 15
+// What bounds it: the MFMAs, 32 of 13.5 ns per 256 scores on a SIMD, and 15
 // adds per score beside them. 32 heads over 2,047 positions: 429 -> 207 us
 // (the FMAs on the VALU, queries broadcast from LDS, before; 264 us with the
 // keys read from memory in the operand layout, 16-byte pieces of 64 lines per
@@ -1937,7 +1937,7 @@ mynah_prefill_softmax(float *scores, uint32_t p0, uint32_t sstride, uint32_t n_h
 // value of a later token touches an earlier one's sum.
 // Workgroups with the most positions start first. Grid (n_kv_heads,
 // ceil(group ceil(T / PV_Q) / 4), 128 / ND), block 256.
-// What bounds it: the MFMAs, 8 of 13.6 ns per 4 positions and 16 queries on a
+// What bounds it: the MFMAs, 8 of 13.5 ns per 4 positions and 16 queries on a
 // SIMD. 32 heads over 2,047 positions: 493 -> 153 us (one VALU chain per
 // lane, probabilities broadcast from LDS, before).
 #define PV_Q 16
@@ -2098,8 +2098,10 @@ MYNAH_DEV void prefill_pv(const float *__restrict__ v_layer, const float *__rest
         uint32_t group) {                                                                     \
         prefill_pv<ND>(v_layer, probs, out, p0, T, sstride, kv_dim, group);                   \
     }
-PV_KERNEL(128, 3)      // 63 positions x 16 heads: 8.4 us, 2,047 x 32: 153 us
-PV_KERNEL(32, 4)       // 63 positions x 16 heads: 5.0 us, 2,047 x 32: 175 us
+// 63 positions x 16 heads 8.4 and 5.0 us (4.2 in the VALU form before), 2,047 x
+// 32 153 and 175. At three waves a SIMD the first spills two registers.
+PV_KERNEL(128, 3)
+PV_KERNEL(32, 4)
 
 // Test hook for the chain property that the two kernels above rest on (no
 // reference counterpart). Per workgroup (one wave) 16 x 4 values of a, 4 x 16

@@ -48,7 +48,7 @@
 // phase hit 16 different bank groups), one barrier per stage.
 //
 // What bounds it: issue. An MFMA of this shape takes 32 cycles of its SIMD
-// (13.7 ns) and does not overlap f32 adds, its own wave's or another's; 16 adds
+// (13.5 ns) and does not overlap f32 adds, its own wave's or another's; 16 adds
 // of registers take 15 ns where two waves alternate (a wave alone issues one
 // instruction every 4 cycles, and waves share two ports, so an odd number of
 // them leaves one idle part of the time; any scalar-register operand doubles

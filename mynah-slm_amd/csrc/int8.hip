@@ -188,13 +188,18 @@ extern "C" __global__ __launch_bounds__(256) void mynah_q4k_gemv_int8(
 // (scale_j, -offset_j) and the tokens' sums as floats are computed into LDS
 // from block headers and sums held in registers a super-block ahead. One
 // barrier per super-block.
-// What bounds it: issue. Per four tiles (1,024 outputs) and sub-block the four
-// i8 MFMAs (27 ns), 16 subtractions (18), 16 v_fmac (24) and the rank-one MFMA
-// (14) do not overlap on a SIMD: about 83 ns, where the form with a conversion
-// and both FMAs on the VALU took about 130. Measured on MI355X with the
-// quantiser, before (64 x 64 tiles, activations as the MFMA's columns) and now:
-// 9728 x 2560 Q4_K, 2047 tokens 347 -> 245 us; 6144 x 2048, 512 tokens 57 ->
-// 38 us; 4096 x 2560 Q5_K, 130 tokens 45 -> 28 us.
+// What bounds it: issue. Per tile (256 outputs) and sub-block an i8 MFMA (7.0
+// ns of its SIMD), 4 subtractions and 8 v_fmac (1.04 each) do not overlap: 19.5
+// ns. The 128 x 128 tile alone has the four tiles a wave that a rank-one MFMA
+// takes (13.5 ns for 16 v_fmac): 18.8. The tile the host picks for 6144 x 2048,
+// 512 tokens is 96 x 128 (three a wave) and for 4096 x 2560, 130 tokens 32 x 32
+// (one): 15 and 3.2 us by these, against calls of 38 and 28 (31 of them the
+// first's kernel). In that they are 9.4 of 17.2 million VALU instructions; unpacking, staging and
+// addresses are the others, about 9 us, and the rest waits for copies and the
+// barrier of each super-block. Measured on MI355X with the
+// quantiser, the form before (64 x 64 tiles, activations as the MFMA's columns,
+// a conversion per dot) and this: 9728 x 2560 Q4_K, 2047 tokens 347 -> 245 us;
+// 6144 x 2048, 512 tokens 57 -> 38 us; 4096 x 2560 Q5_K, 130 tokens 45 -> 28 us.
 // Q5_K (FMT 13, kernels.c:1155-1185 q5_k_quants): the same tiles, the quant
 // bytes at block offset 48 instead of 16, and each lane also holds the 8 qh
 // bytes of its 8 positions: bit j of qh[i] is the fifth bit (+16) of weight
@@ -529,7 +534,8 @@ MYNAH_DEV void gemm_int8(const uint8_t *__restrict__ w, const int8_t *__restrict
 }
 
 // ROWSxTOK: the workgroup's tile, of 16 waves (four per SIMD) where it is
-// large. The tiles the host chooses among, by rows and tokens (int8.c).
+// large. The tiles the host chooses among, by rows and tokens (int8.c). At four
+// waves a SIMD the 128 x 128 tile spills one register (Q4_K) and four (Q5_K).
 #define GEMM_INT8(NAME, FMT, WR, WT, TR, TT, TILE)                                           \
     extern "C" __global__ __launch_bounds__(64 * WR * WT, WR * WT == 16 ? 4 : 2) void        \
         NAME##_##TILE(const uint8_t *__restrict__ w, const int8_t *__restrict__ xq,          \
